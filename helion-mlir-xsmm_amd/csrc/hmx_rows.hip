@@ -2,18 +2,18 @@
 // row sums, row dots, gemv, column sums and elementwise ops.
 //
 // A row (or one (row, group) unit) is read once from HBM with 16-byte loads
-// (`global_load_dwordx4`) into registers, reduced, and written once with
-// non-temporal stores: one HBM read and one write per element, the floor for
-// these ops. Rows of at most 64 vectors take the smallest power-of-two group
-// of lanes that holds them (several rows per wave), rows of up to 128
-// vectors one wave each (four rows per 256-thread workgroup). Longer rows take a whole
-// workgroup of WPR waves (up to 16) holding two or more vectors per lane and
-// combine the per-wave reductions through LDS: a [32768, 4096] f32 softmax
-// runs 32768 workgroups of 8 waves with 8 values per lane, which measures
-// ~25% more bandwidth on gfx950 than one wave holding the 4096-value row (64
-// values per lane, 5 waves per SIMD). Rows longer than the register cache
-// (16 waves x 64 values per lane) stream through the same math in chunks, one
-// wave per row.
+// (`global_load_dwordx4`, at any element alignment) into registers, reduced,
+// and written once with non-temporal stores: one HBM read and one write per
+// element, the floor for these ops. Rows of at most 64 vectors take the
+// smallest power-of-two group of lanes that holds them (several rows per wave),
+// rows of up to 128 vectors one wave each (four rows per 256-thread
+// workgroup). Longer rows take a whole workgroup of as many waves as hold
+// them with two vectors per lane (up to 16 waves, then more vectors per lane)
+// and combine the per-wave reductions through LDS: a [32768, 4096] f32
+// softmax runs 32768 workgroups of 8 waves with 8 values per lane, which
+// measures ~25% more bandwidth on gfx950 than one wave holding the 4096-value
+// row (64 values per lane, 5 waves per SIMD). Rows longer than the register
+// cache stream through the same math in chunks.
 #include <atomic>
 #include <type_traits>
 #include <utility>
@@ -26,7 +26,9 @@ namespace {
 // ---------------------------------------------------------------------------
 // Softmax: max, sum of exp(x - max), then exp(x - max) * (1 / sum), as
 // helion_mlir_utils/normalization.py:47-72 computes it (f32 inside, one
-// rounding), with the row held in registers between the passes. The grid
+// rounding), with the row held in registers between the passes (up to 64
+// values a lane: [512, 50001] f32 47 us, [4000, 20000] bf16 55 us; streamed,
+// 48 and 95 us). The grid
 // holds exactly the rows (tpr > 64: one workgroup per row), so no thread that
 // reaches a barrier has returned early.
 template <typename T, int EPV, int VPL, bool WHOLE>
@@ -36,7 +38,7 @@ __global__ __launch_bounds__(kMaxBlock) void softmax_cached(const T* x, T* y, in
   const RowPos p = row_pos(tpr);
   if (p.row >= m) return;
   float v[VPL * EPV];
-  load_row<T, EPV, VPL, WHOLE>(x + p.row * n, n, p.li, p.tpr, v, -INFINITY);
+  load_row<T, EPV, VPL, WHOLE>(x + p.row * n, (int)n, p.li, p.tpr, v, -INFINITY);
   float mx = -INFINITY;
 #pragma unroll
   for (int i = 0; i < VPL * EPV; ++i) mx = fmaxf(mx, v[i]);
@@ -44,47 +46,65 @@ __global__ __launch_bounds__(kMaxBlock) void softmax_cached(const T* x, T* y, in
   float sum = 0.f;
 #pragma unroll
   for (int i = 0; i < VPL * EPV; ++i) {
+    // Past the row's end v is -inf: its exponential is 0 (or NaN where a NaN
+    // or infinite maximum makes the whole row NaN).
     v[i] = exp_sub(v[i], mx);
-    if (WHOLE || col_of<EPV>(i / EPV, p.li, p.tpr, i % EPV) < n) sum += v[i];
+    sum += v[i];
   }
   sum = row_sum_all(sum, red_sum, tpr);
   const float inv = 1.f / sum;
 #pragma unroll
   for (int i = 0; i < VPL * EPV; ++i) v[i] *= inv;
-  store_row<T, EPV, VPL, WHOLE>(y + p.row * n, n, p.li, p.tpr, v);
+  store_row<T, EPV, VPL, WHOLE>(y + p.row * n, (int)n, p.li, p.tpr, v);
 }
 
+// Rows longer than the register cache: one workgroup of 1024 threads per row,
+// two passes (bound by HBM and, on the second, by the caches: f32 rows of
+// 128000, 512 of them, 710-800 us with a wave per row and three passes, 118
+// us). The first keeps each thread's running maximum and its sum of
+// exp(x - that maximum), rescaled when a later chunk raises the maximum; the
+// threads' pairs then combine to the row's. The second pass walks the row
+// from its end, whose chunks the caches still hold, and writes the results.
+// A thread that has met only -inf keeps base 0, so its exponentials are 0.
 template <typename T, int EPV>
-__global__ __launch_bounds__(kBlock) void softmax_stream(const T* x,
-                                                         T* y, int64_t m,
-                                                         int64_t n) {
-  const int64_t row = unit_index();
-  if (row >= m) return;
-  const int lane = threadIdx.x & (kWave - 1);
-  const T* xr = x + row * n;
-  T* yr = y + row * n;
-  const int64_t step = (int64_t)kWave * EPV;
-  float v[EPV];
-  float mx = -INFINITY;
-  for (int64_t col = (int64_t)lane * EPV; col < n; col += step) {
-    load_chunk<T, EPV>(xr, n, col, v, -INFINITY);
+__global__ __launch_bounds__(kMaxBlock) void softmax_stream(const T* x, T* y, int64_t n) {
+  constexpr int U = 4;  // vectors in flight per thread
+  __shared__ float red_max[kMaxWavesPerRow], red_sum[kMaxWavesPerRow];
+  const T* xr = x + (int64_t)blockIdx.x * n;
+  T* yr = y + (int64_t)blockIdx.x * n;
+  const int64_t step = (int64_t)kMaxBlock * EPV, big = step * U;
+  const int64_t chunks = (n + big - 1) / big, col0 = (int64_t)threadIdx.x * EPV;
+  float v[U][EPV];
+  float mx = -INFINITY, base = 0.f, sum = 0.f;
+  for (int64_t c = 0; c < chunks; ++c) {
+    float top = mx;
 #pragma unroll
-    for (int e = 0; e < EPV; ++e) mx = fmaxf(mx, v[e]);
+    for (int u = 0; u < U; ++u) load_chunk<T, EPV>(xr, n, c * big + u * step + col0, v[u], -INFINITY);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int e = 0; e < EPV; ++e) top = fmaxf(top, v[u][e]);
+    if (top > mx) {
+      if (mx > -INFINITY) sum *= exp_sub(mx, top);
+      mx = base = top;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int e = 0; e < EPV; ++e) sum += exp_sub(v[u][e], base);
   }
-  mx = wave_max(mx);
-  float sum = 0.f;
-  for (int64_t col = (int64_t)lane * EPV; col < n; col += step) {
-    load_chunk<T, EPV>(xr, n, col, v, -INFINITY);
+  const float row_mx = row_max_all(mx, red_max, kMaxBlock);
+  if (mx > -INFINITY) sum *= exp_sub(mx, row_mx);
+  const float inv = 1.f / row_sum_all(sum, red_sum, kMaxBlock);
+  for (int64_t c = chunks - 1; c >= 0; --c) {
 #pragma unroll
-    for (int e = 0; e < EPV; ++e)
-      if (col + e < n) sum += exp_sub(v[e], mx);
-  }
-  const float inv = 1.f / wave_sum(sum);
-  for (int64_t col = (int64_t)lane * EPV; col < n; col += step) {
-    load_chunk<T, EPV>(xr, n, col, v, 0.f);
+    for (int u = 0; u < U; ++u) load_chunk<T, EPV>(xr, n, c * big + u * step + col0, v[u], 0.f);
 #pragma unroll
-    for (int e = 0; e < EPV; ++e) v[e] = exp_sub(v[e], mx) * inv;
-    store_chunk<T, EPV>(yr, n, col, v);
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int e = 0; e < EPV; ++e) v[u][e] = exp_sub(v[u][e], row_mx) * inv;
+      store_chunk<T, EPV>(yr, n, c * big + u * step + col0, v[u]);
+    }
   }
 }
 
@@ -94,13 +114,12 @@ __global__ __launch_bounds__(kBlock) void softmax_stream(const T* x,
 // as x, so its loads are vectors too.
 template <typename T, typename W, int EPV, int VPL, bool WHOLE>
 __global__ __launch_bounds__(kMaxBlock) void rmsnorm_cached(const T* x, const W* __restrict__ w,
-                                                            bool w_vec, T* y, int64_t m,
-                                                            int64_t n, float eps, int tpr) {
+                                                            T* y, int64_t m, int64_t n, float eps, int tpr) {
   __shared__ float red_sum[kMaxWavesPerRow];
   const RowPos p = row_pos(tpr);
   if (p.row >= m) return;
   float v[VPL * EPV];
-  load_row<T, EPV, VPL, WHOLE>(x + p.row * n, n, p.li, p.tpr, v, 0.f);
+  load_row<T, EPV, VPL, WHOLE>(x + p.row * n, (int)n, p.li, p.tpr, v, 0.f);
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < VPL * EPV; ++i) ss = __builtin_fmaf(v[i], v[i], ss);
@@ -110,7 +129,7 @@ __global__ __launch_bounds__(kMaxBlock) void rmsnorm_cached(const T* x, const W*
   for (int j = 0; j < VPL; ++j) {
     float wv[EPV];
     if (w != nullptr) {
-      load_vec_run<W, EPV>(w, n, col_of<EPV>(j, p.li, p.tpr, 0), w_vec, wv);
+      load_vec_run<W, EPV>(w, n, col_of<EPV>(j, p.li, p.tpr, 0), wv);
     } else {
 #pragma unroll
       for (int e = 0; e < EPV; ++e) wv[e] = 1.f;
@@ -118,7 +137,7 @@ __global__ __launch_bounds__(kMaxBlock) void rmsnorm_cached(const T* x, const W*
 #pragma unroll
     for (int e = 0; e < EPV; ++e) v[j * EPV + e] = v[j * EPV + e] * r * wv[e];
   }
-  store_row<T, EPV, VPL, WHOLE>(y + p.row * n, n, p.li, p.tpr, v);
+  store_row<T, EPV, VPL, WHOLE>(y + p.row * n, (int)n, p.li, p.tpr, v);
 }
 
 // RMSNorm of two rows per workgroup (rows of more than 64 threads, one row
@@ -127,16 +146,15 @@ __global__ __launch_bounds__(kMaxBlock) void rmsnorm_cached(const T* x, const W*
 // rmsnorm_cached's (same lanes, same order), so the results are equal.
 template <typename T, typename W, int EPV, int VPL, bool WHOLE>
 __global__ __launch_bounds__(kMaxBlock) void rmsnorm_cached2(const T* x, const W* __restrict__ w,
-                                                             bool w_vec, T* y, int64_t m,
-                                                             int64_t n, float eps, int tpr) {
+                                                             T* y, int64_t m, int64_t n, float eps, int tpr) {
   __shared__ float red_sum[2][kMaxWavesPerRow];
   const int li = (int)threadIdx.x;  // tpr == blockDim.x
   const int64_t r0 = (int64_t)blockIdx.x * 2;
   const bool two = r0 + 1 < m;
   float v0[VPL * EPV], v1[VPL * EPV];
-  load_row<T, EPV, VPL, WHOLE>(x + r0 * n, n, li, tpr, v0, 0.f);
+  load_row<T, EPV, VPL, WHOLE>(x + r0 * n, (int)n, li, tpr, v0, 0.f);
   if (two) {
-    load_row<T, EPV, VPL, WHOLE>(x + (r0 + 1) * n, n, li, tpr, v1, 0.f);
+    load_row<T, EPV, VPL, WHOLE>(x + (r0 + 1) * n, (int)n, li, tpr, v1, 0.f);
   } else {
 #pragma unroll
     for (int i = 0; i < VPL * EPV; ++i) v1[i] = 0.f;
@@ -154,7 +172,7 @@ __global__ __launch_bounds__(kMaxBlock) void rmsnorm_cached2(const T* x, const W
   for (int j = 0; j < VPL; ++j) {
     float wv[EPV];
     if (w != nullptr) {
-      load_vec_run<W, EPV>(w, n, col_of<EPV>(j, li, tpr, 0), w_vec, wv);
+      load_vec_run<W, EPV>(w, n, col_of<EPV>(j, li, tpr, 0), wv);
     } else {
 #pragma unroll
       for (int e = 0; e < EPV; ++e) wv[e] = 1.f;
@@ -165,14 +183,13 @@ __global__ __launch_bounds__(kMaxBlock) void rmsnorm_cached2(const T* x, const W
       v1[j * EPV + e] = v1[j * EPV + e] * q1 * wv[e];
     }
   }
-  store_row<T, EPV, VPL, WHOLE>(y + r0 * n, n, li, tpr, v0);
-  if (two) store_row<T, EPV, VPL, WHOLE>(y + (r0 + 1) * n, n, li, tpr, v1);
+  store_row<T, EPV, VPL, WHOLE>(y + r0 * n, (int)n, li, tpr, v0);
+  if (two) store_row<T, EPV, VPL, WHOLE>(y + (r0 + 1) * n, (int)n, li, tpr, v1);
 }
 
 template <typename T, typename W, int EPV>
 __global__ __launch_bounds__(kBlock) void rmsnorm_stream(const T* x, const W* __restrict__ w,
-                                                         bool w_vec, T* y, int64_t m,
-                                                         int64_t n, float eps) {
+                                                         T* y, int64_t m, int64_t n, float eps) {
   const int64_t row = unit_index();
   if (row >= m) return;
   const int lane = threadIdx.x & (kWave - 1);
@@ -191,7 +208,7 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_stream(const T* x, const W* __
     load_chunk<T, EPV>(xr, n, col, v, 0.f);
     float wv[EPV];
     if (w != nullptr) {
-      load_vec_run<W, EPV>(w, n, col, w_vec, wv);
+      load_vec_run<W, EPV>(w, n, col, wv);
     } else {
 #pragma unroll
       for (int e = 0; e < EPV; ++e) wv[e] = 1.f;
@@ -219,63 +236,72 @@ __device__ __forceinline__ float group_norm_pre(const GroupNormArgs& a, float ce
   return yv;
 }
 
-template <typename T, int EPV, int VPL, bool WHOLE>
-__global__ __launch_bounds__(kMaxBlock) void group_norm_cached(const T* x, T* y, GroupNormArgs a,
-                                                               int tpr) {
+// GroupNorm of units that group_norm_rows does not take (groups of any size,
+// rows no power of two fills): `tpr` threads per (row, group) unit, each
+// workgroup bound to gpw neighbouring groups of rpw rows at a time and walking
+// the rows with w, b and the extra vector of its groups' channels in
+// registers, as group_norm_rows does with whole rows. Loaded again for every
+// unit, f32 w and b move four times a bf16 row's bytes: LayerNorm of
+// [16384, 5120] bf16 105 -> 75 us, GroupNorm-32 of it 116 -> 86 us.
+// Walked rows reuse the reduction slots: a slot of one kind is written again
+// only after the barrier of the other kind, which its readers have reached.
+template <typename T, int EPV, int VPL, bool WHOLE, bool EXTRA>
+__global__ __launch_bounds__(kMaxBlock) void group_norm_walk(const T* x, T* y, GroupNormArgs a, int64_t rows,
+                                                             int tpr, int gpw, int rpw) {
   __shared__ float red_mean[kMaxWavesPerRow], red_var[kMaxWavesPerRow];
-  const RowPos p = row_pos(tpr);
-  const int64_t unit = p.row;
-  if (unit >= a.units) return;
-  const int64_t g = unit % a.groups;
+  const int slot = tpr <= kWave ? (int)threadIdx.x / tpr : 0;
+  const int li = tpr <= kWave ? (int)threadIdx.x % tpr : (int)threadIdx.x;
+  const int64_t g = (int64_t)blockIdx.x * gpw + slot % gpw;
+  int64_t row = (int64_t)blockIdx.y * rpw + slot / gpw;
+  // tpr > 64: the whole workgroup is one unit (gpw = rpw = 1) and leaves
+  // together.
+  if (slot / gpw >= rpw || g >= a.groups || row >= rows) return;
   const int64_t n = a.gs;
-  float v[VPL * EPV];
-  load_row<T, EPV, VPL, WHOLE>(x + unit * n, n, p.li, p.tpr, v, 0.f);
-  float s = 0.f;
-#pragma unroll
-  for (int i = 0; i < VPL * EPV; ++i) s += v[i];
-  const float mean = row_sum_all(s, red_mean, tpr) / (float)n;
-  float q = 0.f;
-#pragma unroll
-  for (int i = 0; i < VPL * EPV; ++i) {
-    const float c = v[i] - mean;
-    if (WHOLE || col_of<EPV>(i / EPV, p.li, p.tpr, i % EPV) < n) q += c * c;
-  }
-  const float r = rsqrtf(row_sum_all(q, red_var, tpr) / (float)n + a.eps);
-  const bool prog = a.act == HMX_EPI_PROGRAM;
-  float ex[VPL * EPV];
+  float wv[VPL * EPV], bv[VPL * EPV], ev[EXTRA ? VPL * EPV : 1];
 #pragma unroll
   for (int j = 0; j < VPL; ++j) {
-    if constexpr (EPV > 1) {
-      const int64_t col0 = col_of<EPV>(j, p.li, p.tpr, 0);
-      if (a.vec_ok && (WHOLE || col0 + EPV <= n)) {
-        // The same arithmetic as group_norm_pre, on whole vectors of w, b, extra.
-        float wv[EPV], bv[EPV], ev[EPV];
-        load_vec_any<EPV>(a.w, a.vec_dtype, g * n + col0, wv, 1.f);
-        load_vec_any<EPV>(a.b, a.vec_dtype, g * n + col0, bv, 0.f);
-        load_vec_any<EPV>(a.extra_op != HMX_EXTRA_NONE || prog ? a.extra : nullptr, a.vec_dtype, g * n + col0,
-                          ev, 0.f);
+    const int64_t col = g * n + col_of<EPV>(j, li, tpr, 0), end = (g + 1) * n;
+    float t[EPV];
+    load_vec_any<EPV>(a.w, a.vec_dtype, end, col, t, 1.f);
 #pragma unroll
-        for (int e = 0; e < EPV; ++e) {
-          float yv = (v[j * EPV + e] - mean) * r * wv[e];
-          yv += bv[e];
-          if (!prog && a.extra_op == HMX_EXTRA_ADD) yv += ev[e];
-          if (!prog && a.extra_op == HMX_EXTRA_MUL) yv *= ev[e];
-          v[j * EPV + e] = yv;
-          ex[j * EPV + e] = ev[e];
-        }
-        continue;
-      }
-    }
+    for (int e = 0; e < EPV; ++e) wv[j * EPV + e] = t[e];
+    load_vec_any<EPV>(a.b, a.vec_dtype, end, col, t, 0.f);
 #pragma unroll
-    for (int e = 0; e < EPV; ++e) {
-      const int64_t col = col_of<EPV>(j, p.li, p.tpr, e);
-      ex[j * EPV + e] = 0.f;
-      if (WHOLE || col < n)
-        v[j * EPV + e] = group_norm_pre(a, v[j * EPV + e] - mean, r, g * n + col, ex[j * EPV + e]);
+    for (int e = 0; e < EPV; ++e) bv[j * EPV + e] = t[e];
+    if constexpr (EXTRA) {
+      load_vec_any<EPV>(a.extra, a.vec_dtype, end, col, t, 0.f);
+#pragma unroll
+      for (int e = 0; e < EPV; ++e) ev[j * EPV + e] = t[e];
     }
   }
-  group_norm_finish<VPL * EPV, false>(a, v, ex);
-  store_row<T, EPV, VPL, WHOLE>(y + unit * n, n, p.li, p.tpr, v);
+  for (; row < rows; row += (int64_t)gridDim.y * rpw) {
+    const int64_t off = (row * a.groups + g) * n;
+    float v[VPL * EPV];
+    load_row<T, EPV, VPL, WHOLE>(x + off, (int)n, li, tpr, v, 0.f);
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < VPL * EPV; ++i) s += v[i];
+    const float mean = row_sum_all(s, red_mean, tpr) / (float)n;
+    float q = 0.f;
+#pragma unroll
+    for (int i = 0; i < VPL * EPV; ++i) {
+      const float c = v[i] - mean;
+      if (WHOLE || col_of<EPV>(i / EPV, li, tpr, i % EPV) < n) q += c * c;
+    }
+    const float r = rsqrtf(row_sum_all(q, red_var, tpr) / (float)n + a.eps);
+#pragma unroll
+    for (int i = 0; i < VPL * EPV; ++i) {
+      float yv = (v[i] - mean) * r * wv[i];
+      yv += bv[i];
+      if constexpr (EXTRA) {
+        if (a.extra_op == HMX_EXTRA_ADD) yv += ev[i];
+        if (a.extra_op == HMX_EXTRA_MUL) yv *= ev[i];
+      }
+      v[i] = yv;
+    }
+    group_norm_finish<VPL * EPV, false>(a, v, v);
+    store_row<T, EPV, VPL, WHOLE>(y + off, (int)n, li, tpr, v);
+  }
 }
 
 // Whole-row GroupNorm (body in hmx_rows_common.hpp). PROG: the epilogue is
@@ -356,7 +382,7 @@ __global__ __launch_bounds__(kBlock) void row_reduce(const T* x,
       for (int e = 0; e < EPV; ++e) s += v[e];
     } else if constexpr (MODE == 1) {
       float u[EPV];
-      load_f32_run<EPV>((const float*)vec, n, col, u);
+      load_vec_run<float, EPV>((const float*)vec, n, col, u);
 #pragma unroll
       for (int e = 0; e < EPV; ++e) s += v[e] * u[e];
     } else {
@@ -487,20 +513,24 @@ __global__ __launch_bounds__(256) void elementwise_kernel(const T* x,
 // ---------------------------------------------------------------------------
 // Host dispatch.
 
-// Layout of a cached row kernel for rows of n elements in vectors of epv:
-// rows of at most 64 vectors take the smallest power-of-two lane group that
-// holds them (one vector per lane; e.g. GroupNorm's 128-channel bf16 groups:
-// four groups per wave); rows of up to 128 vectors one wave (two vectors per
-// lane); longer rows a workgroup of tpr / 64 waves with two vectors per
-// lane, doubling up to 16 waves, then more vectors per lane up to kMaxPerLane
-// values. vpl == 0: the row needs the streaming kernel.
+// Layout of a cached row kernel for rows of n elements in vectors of epv, at
+// most max_per_lane values per lane: rows of at most 64 vectors take the
+// smallest power-of-two lane group that holds them (one vector per lane; e.g.
+// GroupNorm's 128-channel bf16 groups: four groups per wave); rows of up to
+// 128 vectors one wave (two vectors per lane); longer rows a workgroup of as
+// many waves as hold them with two vectors per lane (a power of two of waves
+// left up to half the lanes of the second vector idle: softmax of
+// [8192, 5120] bf16 38.5 -> 25.7 us), past 16 waves with more vectors per lane.
+// vpl == 0: the row needs the streaming kernel.
 struct RowShape {
-  int tpr;  // threads per row (a power of two; up to 64 * kMaxWavesPerRow)
+  int tpr;  // threads per row (a power of two up to 64, else a multiple of 64 up to 64 * kMaxWavesPerRow)
   int vpl;
-  bool whole;  // n == tpr * vpl * epv with 16-byte vectors: no guards
+  bool whole;  // n == tpr * vpl * epv: no guards
 };
 
-RowShape row_shape(int64_t n, int epv) {
+constexpr int kVpls[] = {1, 2, 3, 4, 6, 8, 12, 16};
+
+RowShape row_shape(int64_t n, int epv, int max_per_lane = kMaxPerLane) {
   const int64_t vecs = ceil_div(n, epv);
   RowShape r{kWave, 0, false};
   if (vecs <= kWave) {
@@ -511,15 +541,14 @@ RowShape row_shape(int64_t n, int epv) {
   } else if (vecs <= 2 * kWave) {
     r.vpl = 2;
   } else {
-    r.tpr = 2 * kWave;
-    while (r.tpr < kMaxWavesPerRow * kWave && (int64_t)r.tpr * 2 < vecs) r.tpr *= 2;
-    for (int vpl = 2; vpl * epv <= kMaxPerLane; vpl *= 2)
-      if ((int64_t)r.tpr * vpl >= vecs) {
+    r.tpr = (int)std::min<int64_t>(ceil_div(vecs, 2 * kWave), kMaxWavesPerRow) * kWave;
+    for (int vpl : kVpls)
+      if (vpl >= 2 && vpl * epv <= max_per_lane && (int64_t)r.tpr * vpl >= vecs) {
         r.vpl = vpl;
         break;
       }
   }
-  r.whole = r.vpl > 0 && epv > 1 && n == (int64_t)r.tpr * r.vpl * epv;
+  r.whole = r.vpl > 0 && n == (int64_t)r.tpr * r.vpl * epv;
   return r;
 }
 
@@ -542,23 +571,27 @@ bool rms_two_rows() {
 template <int V>
 using IntC = std::integral_constant<int, V>;
 
-// Calls f(IntC<VPL>) for the runtime vpl (a power of two, VPL * EPV <= kMaxPerLane).
-template <int EPV, typename F>
+// Calls f(IntC<VPL>) for the runtime vpl (one of kVpls, VPL * EPV <= MAX).
+template <int EPV, int MAX = kMaxPerLane, typename F>
 void with_vpl(int vpl, F&& f) {
   switch (vpl) {
     case 1: f(IntC<1>{}); break;
     case 2: f(IntC<2>{}); break;
-    case 4: if constexpr (4 * EPV <= kMaxPerLane) f(IntC<4>{}); break;
-    case 8: if constexpr (8 * EPV <= kMaxPerLane) f(IntC<8>{}); break;
-    case 16: if constexpr (16 * EPV <= kMaxPerLane) f(IntC<16>{}); break;
+    case 3: if constexpr (3 * EPV <= MAX) f(IntC<3>{}); break;
+    case 4: if constexpr (4 * EPV <= MAX) f(IntC<4>{}); break;
+    case 6: if constexpr (6 * EPV <= MAX) f(IntC<6>{}); break;
+    case 8: if constexpr (8 * EPV <= MAX) f(IntC<8>{}); break;
+    case 12: if constexpr (12 * EPV <= MAX) f(IntC<12>{}); break;
+    case 16: if constexpr (16 * EPV <= MAX) f(IntC<16>{}); break;
   }
 }
 
 // Calls f(IntC<VPL>, bool_constant<WHOLE>) for a cached row shape.
-template <int EPV, typename F>
+template <int EPV, int MAX = kMaxPerLane, typename F>
 void with_shape(const RowShape& r, F&& f) {
-  with_vpl<EPV>(r.vpl, [&](auto vpl_c) {
-    if constexpr (EPV > 1) {
+  with_vpl<EPV, MAX>(r.vpl, [&](auto vpl_c) {
+    // Rows past four vectors per lane are few and long: guards cost nothing.
+    if constexpr (decltype(vpl_c)::value <= 4) {
       if (r.whole) {
         f(vpl_c, std::true_type{});
         return;
@@ -568,22 +601,11 @@ void with_shape(const RowShape& r, F&& f) {
   });
 }
 
-// Calls f(T*, IntC<EPV>) for the dtype and whether 16-byte vectors apply.
+// Calls f(T*, IntC<EPV>) for the dtype, EPV elements per 16-byte vector.
 template <typename F>
-void with_type(int dtype, bool vec, F&& f) {
-  if (dtype == HMX_DTYPE_BF16) {
-    if (vec) f((uint16_t*)nullptr, IntC<8>{});
-    else f((uint16_t*)nullptr, IntC<1>{});
-  } else {
-    if (vec) f((float*)nullptr, IntC<4>{});
-    else f((float*)nullptr, IntC<1>{});
-  }
-}
-
-// Whether rows of `n` elements starting at `p` (and `q`) keep 16-byte alignment.
-bool rows_vectorizable(const void* p, const void* q, int64_t n, int dtype) {
-  const int64_t epv = 16 / dtype_bytes(dtype);
-  return aligned16(p) && aligned16(q) && n % epv == 0;
+void with_type(int dtype, F&& f) {
+  if (dtype == HMX_DTYPE_BF16) f((uint16_t*)nullptr, IntC<8>{});
+  else f((float*)nullptr, IntC<4>{});
 }
 
 dim3 unit_grid(int64_t units) { return dim3((unsigned)ceil_div(units, kRowsPerBlock)); }
@@ -594,9 +616,8 @@ dim3 unit_grid(int64_t units) { return dim3((unsigned)ceil_div(units, kRowsPerBl
 // that none waits for another to finish.
 template <auto Kernel>
 int resident_blocks(int block) {
-  static std::atomic<int> known[5];  // block = 64 << i
-  int i = 0;
-  while (i < 4 && (kWave << i) < block) ++i;
+  static std::atomic<int> known[kMaxWavesPerRow];  // by waves per workgroup
+  const int i = block / kWave - 1;
   int b = known[i].load(std::memory_order_relaxed);
   if (b > 0) return b;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, Kernel, block, 0) != hipSuccess || b < 1) {
@@ -626,15 +647,15 @@ int hmx_softmax_rows(int dtype, const void* x, void* y, int64_t m, int64_t n,
   HMX_REQUIRE(m <= kMaxGrid, "softmax: too many rows");
   if (m == 0) return HMX_OK;
   auto s = (hipStream_t)stream;
-  with_type(dtype, rows_vectorizable(x, y, n, dtype), [&](auto tp, auto epv_c) {
+  with_type(dtype, [&](auto tp, auto epv_c) {
     using T = std::remove_pointer_t<decltype(tp)>;
     constexpr int EPV = decltype(epv_c)::value;
-    const RowShape r = row_shape(n, EPV);
+    const RowShape r = row_shape(n, EPV, kSoftmaxMaxPerLane);
     if (r.vpl == 0) {
-      launch(softmax_stream<T, EPV>, unit_grid(m), kBlock, s, (const T*)x, (T*)y, m, n);
+      launch(softmax_stream<T, EPV>, dim3((unsigned)m), kMaxBlock, s, (const T*)x, (T*)y, n);
       return;
     }
-    with_shape<EPV>(r, [&](auto vpl_c, auto whole_c) {
+    with_shape<EPV, kSoftmaxMaxPerLane>(r, [&](auto vpl_c, auto whole_c) {
       launch(softmax_cached<T, EPV, decltype(vpl_c)::value, decltype(whole_c)::value>,
              dim3((unsigned)row_grid(m, r)), row_block(r), s, (const T*)x, (T*)y, m, n, r.tpr);
     });
@@ -652,16 +673,14 @@ int hmx_rmsnorm_rows(int dtype, const void* x, const void* w, int w_dtype, void*
   HMX_REQUIRE(m <= kMaxGrid, "rms_norm: too many rows");
   if (m == 0) return HMX_OK;
   auto s = (hipStream_t)stream;
-  const bool w_vec = aligned16(w);
-  with_type(dtype, rows_vectorizable(x, y, n, dtype), [&](auto tp, auto epv_c) {
+  with_type(dtype, [&](auto tp, auto epv_c) {
     using T = std::remove_pointer_t<decltype(tp)>;
     constexpr int EPV = decltype(epv_c)::value;
     auto with_weight = [&](auto wp) {
       using W = std::remove_pointer_t<decltype(wp)>;
       const RowShape r = row_shape(n, EPV);
       if (r.vpl == 0) {
-        launch(rmsnorm_stream<T, W, EPV>, unit_grid(m), kBlock, s, (const T*)x, (const W*)w, w_vec,
-               (T*)y, m, n, eps);
+        launch(rmsnorm_stream<T, W, EPV>, unit_grid(m), kBlock, s, (const T*)x, (const W*)w, (T*)y, m, n, eps);
         return;
       }
       with_shape<EPV>(r, [&](auto vpl_c, auto whole_c) {
@@ -671,10 +690,10 @@ int hmx_rmsnorm_rows(int dtype, const void* x, const void* w, int w_dtype, void*
         // f32 rows measured slower that way (169 -> 177 us).
         if (r.tpr > kWave && sizeof(T) == 2 && rms_two_rows())
           launch(rmsnorm_cached2<T, W, EPV, VPLc, WH>, dim3((unsigned)ceil_div(m, 2)), row_block(r), s,
-                 (const T*)x, (const W*)w, w_vec, (T*)y, m, n, eps, r.tpr);
+                 (const T*)x, (const W*)w, (T*)y, m, n, eps, r.tpr);
         else
           launch(rmsnorm_cached<T, W, EPV, VPLc, WH>, dim3((unsigned)row_grid(m, r)), row_block(r), s,
-                 (const T*)x, (const W*)w, w_vec, (T*)y, m, n, eps, r.tpr);
+                 (const T*)x, (const W*)w, (T*)y, m, n, eps, r.tpr);
       });
     };
     if (w != nullptr && w_dtype == HMX_DTYPE_BF16)
@@ -718,63 +737,61 @@ int hmx_group_norm_rows(int dtype, const void* x, const void* w, const void* b,
   a.act = activation;
   a.act_arg = activation_arg;
   a.prog = prog;
-  a.vec_ok = aligned16(w) && aligned16(b) && aligned16(extra);
   auto s = (hipStream_t)stream;
-  with_type(dtype, rows_vectorizable(x, y, group_size, dtype), [&](auto tp, auto epv_c) {
+  with_type(dtype, [&](auto tp, auto epv_c) {
     using T = std::remove_pointer_t<decltype(tp)>;
     constexpr int EPV = decltype(epv_c)::value;
     const RowShape r = row_shape(group_size, EPV);
-    if constexpr (EPV > 1) {
-      // Whole rows in registers when the row fits and each group is one run
-      // of aligned lanes (or the whole row): w, b and extra stay resident.
-      const int64_t row_n = groups * group_size;
-      const RowShape rr = row_shape(row_n, EPV);
-      const int64_t gv = group_size / EPV;
-      const bool one = groups == 1;
-      // A program's interpreter needs more than the 128 VGPRs of a
-      // 1024-thread workgroup: its kernels are built for rows of at most
-      // kProgBlock threads.
-      const bool fits = activation != HMX_EPI_PROGRAM || row_block(rr) <= (unsigned)kProgBlock;
-      const bool whole_rows = a.vec_ok && rr.vpl > 0 && rr.whole && (one || ((gv & (gv - 1)) == 0 && gv <= rr.tpr));
-      // A program compiled into the kernel at run time: no interpreter, so
-      // every whole-row shape (workgroups of up to 16 waves) takes it.
-      if (whole_rows && activation == HMX_EPI_PROGRAM &&
-          launch_group_norm_jit(std::is_same_v<T, uint16_t>, x, y, a, m, rr.tpr, (int)gv, EPV, rr.vpl, one,
-                                extra != nullptr, row_block(rr), rr.tpr <= kWave ? (int)(kBlock / rr.tpr) : 1,
-                                current_device_shape().cus, s) == HMX_OK)
-        return;
-      if (whole_rows && fits) {
-        const int rpb = rr.tpr <= kWave ? (int)(kBlock / rr.tpr) : 1;
-        const unsigned block = row_block(rr);
-        with_vpl<EPV>(rr.vpl, [&](auto vpl_c) {
-          constexpr int VPL = decltype(vpl_c)::value;
-          auto go = [&](auto one_c, auto extra_c, auto prog_c) {
-            constexpr auto kernel = &group_norm_rows<T, EPV, VPL, decltype(one_c)::value, decltype(extra_c)::value,
-                                                     decltype(prog_c)::value>;
-            // As many workgroups as the GPU holds at once, each walking rows
-            // blockIdx, blockIdx + grid, ...
-            const int64_t resident = (int64_t)resident_blocks<kernel>((int)block) * current_device_shape().cus;
-            launch(kernel, dim3((unsigned)std::min(ceil_div(m, rpb), resident)), block, s, (const T*)x, (T*)y, a,
-                   m, rr.tpr, (int)gv);
-          };
-          // With a program, EXTRA: an extra operand is given (the program
-          // reads it); else: an extra op applies.
-          const bool program = activation == HMX_EPI_PROGRAM;
-          const bool has_extra = program ? extra != nullptr : extra_op != HMX_EXTRA_NONE;
-          auto go2 = [&](auto one_c) {
-            if (program) {
-              if (has_extra) go(one_c, std::true_type{}, std::true_type{});
-              else go(one_c, std::false_type{}, std::true_type{});
-            } else {
-              if (has_extra) go(one_c, std::true_type{}, std::false_type{});
-              else go(one_c, std::false_type{}, std::false_type{});
-            }
-          };
-          if (one) go2(std::true_type{});
-          else go2(std::false_type{});
-        });
-        return;
-      }
+    // Whole rows in registers when the row fits and each group is one run
+    // of aligned lanes (or the whole row): w, b and extra stay resident.
+    const int64_t row_n = groups * group_size;
+    const RowShape rr = row_shape(row_n, EPV);
+    const int64_t gv = group_size / EPV;
+    const bool one = groups == 1;
+    // A program's interpreter needs more than the 128 VGPRs of a
+    // 1024-thread workgroup: its kernels are built for rows of at most
+    // kProgBlock threads.
+    const bool fits = activation != HMX_EPI_PROGRAM || row_block(rr) <= (unsigned)kProgBlock;
+    const bool whole_rows = rr.vpl > 0 && rr.whole &&
+                            (one || (group_size % EPV == 0 && (gv & (gv - 1)) == 0 && gv <= rr.tpr && rr.tpr % gv == 0));
+    // A program compiled into the kernel at run time: no interpreter, so
+    // every whole-row shape (workgroups of up to 16 waves) takes it.
+    if (whole_rows && activation == HMX_EPI_PROGRAM &&
+        launch_group_norm_jit(std::is_same_v<T, uint16_t>, x, y, a, m, rr.tpr, (int)gv, EPV, rr.vpl, one,
+                              extra != nullptr, row_block(rr), rr.tpr <= kWave ? (int)(kBlock / rr.tpr) : 1,
+                              current_device_shape().cus, s) == HMX_OK)
+      return;
+    if (whole_rows && fits) {
+      const int rpb = rr.tpr <= kWave ? (int)(kBlock / rr.tpr) : 1;
+      const unsigned block = row_block(rr);
+      with_vpl<EPV>(rr.vpl, [&](auto vpl_c) {
+        constexpr int VPL = decltype(vpl_c)::value;
+        auto go = [&](auto one_c, auto extra_c, auto prog_c) {
+          constexpr auto kernel = &group_norm_rows<T, EPV, VPL, decltype(one_c)::value, decltype(extra_c)::value,
+                                                   decltype(prog_c)::value>;
+          // As many workgroups as the GPU holds at once, each walking rows
+          // blockIdx, blockIdx + grid, ...
+          const int64_t resident = (int64_t)resident_blocks<kernel>((int)block) * current_device_shape().cus;
+          launch(kernel, dim3((unsigned)std::min(ceil_div(m, rpb), resident)), block, s, (const T*)x, (T*)y, a,
+                 m, rr.tpr, (int)gv);
+        };
+        // With a program, EXTRA: an extra operand is given (the program
+        // reads it); else: an extra op applies.
+        const bool program = activation == HMX_EPI_PROGRAM;
+        const bool has_extra = program ? extra != nullptr : extra_op != HMX_EXTRA_NONE;
+        auto go2 = [&](auto one_c) {
+          if (program) {
+            if (has_extra) go(one_c, std::true_type{}, std::true_type{});
+            else go(one_c, std::false_type{}, std::true_type{});
+          } else {
+            if (has_extra) go(one_c, std::true_type{}, std::false_type{});
+            else go(one_c, std::false_type{}, std::false_type{});
+          }
+        };
+        if (one) go2(std::true_type{});
+        else go2(std::false_type{});
+      });
+      return;
     }
     if (activation == HMX_EPI_PROGRAM) {
       // Programs on rows the whole-row kernel does not take run in the
@@ -787,9 +804,24 @@ int hmx_group_norm_rows(int dtype, const void* x, const void* w, const void* b,
       launch(group_norm_stream<T, EPV, false>, unit_grid(units), kBlock, s, (const T*)x, (T*)y, a);
       return;
     }
+    // A workgroup's units: neighbouring groups of one row, then (fewer groups
+    // than units) of the next rows; as many workgroups as the GPU holds at
+    // once share the rows out.
+    const int upw = r.tpr <= kWave ? kBlock / r.tpr : 1;
+    const int gpw = (int)std::min<int64_t>(groups, upw), rpw = upw / gpw;
+    const int64_t across = ceil_div(groups, gpw);
     with_shape<EPV>(r, [&](auto vpl_c, auto whole_c) {
-      launch(group_norm_cached<T, EPV, decltype(vpl_c)::value, decltype(whole_c)::value>,
-             dim3((unsigned)row_grid(units, r)), row_block(r), s, (const T*)x, (T*)y, a, r.tpr);
+      auto go = [&](auto extra_c) {
+        constexpr auto kernel =
+            &group_norm_walk<T, EPV, decltype(vpl_c)::value, decltype(whole_c)::value, decltype(extra_c)::value>;
+        const int64_t resident = (int64_t)resident_blocks<kernel>((int)row_block(r)) * current_device_shape().cus;
+        const int64_t down = std::min<int64_t>(std::min<int64_t>(ceil_div(m, rpw), 65535),
+                                               std::max<int64_t>(1, resident / across));
+        launch(kernel, dim3((unsigned)across, (unsigned)down), row_block(r), s, (const T*)x, (T*)y, a, m, r.tpr,
+               gpw, rpw);
+      };
+      if (extra_op != HMX_EXTRA_NONE) go(std::true_type{});
+      else go(std::false_type{});
     });
   });
   return check_launch("group_norm");
@@ -809,9 +841,7 @@ static int row_reduce_launch(const char* name, int mode, int dtype, const void* 
   HMX_REQUIRE(m <= ((int64_t)1 << 31) * kRowsPerBlock, "%s: too many rows", name);
   if (m == 0) return HMX_OK;
   auto s = (hipStream_t)stream;
-  bool vec_ok = rows_vectorizable(x, x, n, dtype);
-  if (mode != 0) vec_ok = vec_ok && aligned16(vec);
-  with_type(dtype, vec_ok, [&](auto tp, auto epv_c) {
+  with_type(dtype, [&](auto tp, auto epv_c) {
     using T = std::remove_pointer_t<decltype(tp)>;
     constexpr int EPV = decltype(epv_c)::value;
     if (mode == 0)
@@ -874,7 +904,7 @@ int hmx_column_sum(int dtype, const void* x, float* y, int64_t m, int64_t n, voi
               (long long)need, (long long)workspace_bytes);
   auto s = (hipStream_t)stream;
   float* part = chunks > 1 ? (float*)workspace : y;
-  with_type(dtype, rows_vectorizable(x, x, n, dtype), [&](auto tp, auto epv_c) {
+  with_type(dtype, [&](auto tp, auto epv_c) {
     using T = std::remove_pointer_t<decltype(tp)>;
     constexpr int EPV = decltype(epv_c)::value;
     // The fewest threads across (8 to 64) whose vectors span the row.
@@ -903,8 +933,7 @@ int hmx_elementwise(int op, int dtype, const void* x, void* y, int64_t numel, fl
   HMX_REQUIRE(x && y, "elementwise: null operand");
   if (numel == 0) return HMX_OK;
   auto s = (hipStream_t)stream;
-  const bool vec = aligned16(x) && aligned16(y);
-  with_type(dtype, vec, [&](auto tp, auto epv_c) {
+  with_type(dtype, [&](auto tp, auto epv_c) {
     using T = std::remove_pointer_t<decltype(tp)>;
     constexpr int EPV = decltype(epv_c)::value;
     const int64_t blocks = std::min<int64_t>(ceil_div(numel, 256 * EPV), 8192);

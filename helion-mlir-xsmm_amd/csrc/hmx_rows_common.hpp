@@ -31,9 +31,6 @@ struct GroupNormArgs {
   int act;
   float act_arg;
   hmx_program prog;  // act == HMX_EPI_PROGRAM: the whole epilogue, y = prog(value, extra)
-  // w, b and extra are 16-byte aligned: with vectorizable rows (gs a
-  // multiple of EPV), each row vector's EPV channels load as one piece.
-  bool vec_ok;
 };
 
 #ifndef __HIPCC_RTC__
@@ -56,6 +53,9 @@ constexpr int kBlock = kRowsPerBlock * kWave;
 // kernel fits a 1024-thread workgroup (128 VGPRs per lane at most) without
 // spilling. Rows of up to 16 waves x 64 lanes x 16 = 16384 values are cached.
 constexpr int kMaxPerLane = 16;
+// Softmax keeps nothing but the row, so its lanes hold up to 64 values: rows
+// of up to 65536 are cached.
+constexpr int kSoftmaxMaxPerLane = 64;
 // Waves of a workgroup that share one row.
 constexpr int kMaxWavesPerRow = 16;
 constexpr int kMaxBlock = kMaxWavesPerRow * kWave;
@@ -64,56 +64,60 @@ constexpr int kMaxBlock = kMaxWavesPerRow * kWave;
 constexpr int kProgBlock = 8 * kWave;
 
 // ---------------------------------------------------------------------------
+// 16 bytes at an address that keeps only its element type's alignment: rows of
+// any length are read and written as vectors (gfx950 takes 16-byte global
+// accesses at any element address; only the pieces that cross a cache line
+// cost a second request). Element-wise access of the same rows ran at a
+// quarter of the bandwidth: softmax of [24000, 501] bf16 32.6 -> 14.5 us,
+// RMSNorm of [16384, 3001] bf16 118 -> 42 us.
+typedef uint32_t u32x4_any_t __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ uint4 load16(const void* p) {
+  const u32x4_any_t v = *reinterpret_cast<const u32x4_any_t*>(p);
+  return make_uint4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ uint4 load16_nt(const void* p) {
+  const u32x4_any_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any_t*>(p));
+  return make_uint4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ void store16_row(void* p, const uint4& v) {
+  __builtin_nontemporal_store(u32x4_any_t{v.x, v.y, v.z, v.w}, reinterpret_cast<u32x4_any_t*>(p));
+}
+
 // Row access. `tpr` threads share a row; thread `li` of them holds, as its
 // j-th vector, columns [(j * tpr + li) * EPV, ... + EPV): for each j the
 // threads read one contiguous tpr * EPV run, so every load instruction is
 // fully coalesced.
 // WHOLE: n == tpr * VPL * EPV, every vector is in the row (no guards).
 template <typename T, int EPV, int VPL, bool WHOLE = false>
-__device__ __forceinline__ void load_row(const T* __restrict__ p, int64_t n, int li, int tpr,
+__device__ __forceinline__ void load_row(const T* __restrict__ p, int n, int li, int tpr,
                                          float (&v)[VPL * EPV], float fill) {
 #pragma unroll
   for (int j = 0; j < VPL; ++j) {
-    const int64_t col = ((int64_t)j * tpr + li) * EPV;
-    if constexpr (EPV > 1) {
-      if (WHOLE || col + EPV <= n) {
-        uint4 raw;
-        if constexpr (std::is_same_v<T, float>) {
-          // f32 rows: non-temporal loads measure 2-3% more bandwidth on
-          // [32768, 4096] softmax/RMSNorm; for bf16 rows they cost 8-12%.
-          const u32x4_t nt = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p + col));
-          raw = make_uint4(nt[0], nt[1], nt[2], nt[3]);
-        } else {
-          raw = *reinterpret_cast<const uint4*>(p + col);
-        }
-        Elem<T>::unpack(raw, &v[j * EPV]);
-      } else {
-#pragma unroll
-        for (int e = 0; e < EPV; ++e)
-          v[j * EPV + e] = (col + e < n) ? Elem<T>::load(p + col + e) : fill;
-      }
+    const int col = (j * tpr + li) * EPV;
+    if (WHOLE || col + EPV <= n) {
+      // f32 rows: non-temporal loads measure 2-3% more bandwidth on
+      // [32768, 4096] softmax/RMSNorm; for bf16 rows they cost 8-12%.
+      const uint4 raw = std::is_same_v<T, float> ? load16_nt(p + col) : load16(p + col);
+      Elem<T>::unpack(raw, &v[j * EPV]);
     } else {
-      v[j] = col < n ? Elem<T>::load(p + col) : fill;
+#pragma unroll
+      for (int e = 0; e < EPV; ++e) v[j * EPV + e] = (col + e < n) ? Elem<T>::load(p + col + e) : fill;
     }
   }
 }
 
 template <typename T, int EPV, int VPL, bool WHOLE = false>
-__device__ __forceinline__ void store_row(T* __restrict__ p, int64_t n, int li, int tpr,
+__device__ __forceinline__ void store_row(T* __restrict__ p, int n, int li, int tpr,
                                           const float (&v)[VPL * EPV]) {
 #pragma unroll
   for (int j = 0; j < VPL; ++j) {
     const int64_t col = ((int64_t)j * tpr + li) * EPV;
-    if constexpr (EPV > 1) {
-      if (WHOLE || col + EPV <= n) {
-        store16_stream(p + col, Elem<T>::pack(&v[j * EPV]));
-      } else {
-#pragma unroll
-        for (int e = 0; e < EPV; ++e)
-          if (col + e < n) Elem<T>::store(p + col + e, v[j * EPV + e]);
-      }
+    if (WHOLE || col + EPV <= n) {
+      store16_row(p + col, Elem<T>::pack(&v[j * EPV]));
     } else {
-      if (col < n) Elem<T>::store(p + col, v[j]);
+#pragma unroll
+      for (int e = 0; e < EPV; ++e)
+        if (col + e < n) Elem<T>::store(p + col + e, v[j * EPV + e]);
     }
   }
 }
@@ -124,10 +128,10 @@ __device__ __forceinline__ int64_t col_of(int j, int li, int tpr, int e) {
   return ((int64_t)j * tpr + li) * EPV + e;
 }
 
-// Where a thread of a cached-row kernel sits: `tpr` threads per row, a power
-// of two. tpr <= 64: 64 / tpr rows per wave (aligned lane groups) and
-// blockDim.x / tpr rows per workgroup; tpr > 64: tpr / 64 waves per row, one
-// row per workgroup.
+// Where a thread of a cached-row kernel sits. tpr <= 64 threads per row (a
+// power of two): 64 / tpr rows per wave (aligned lane groups) and
+// blockDim.x / tpr rows per workgroup; tpr > 64 (a multiple of 64): tpr / 64
+// waves per row, one row per workgroup.
 struct RowPos {
   int64_t row;
   int li;   // index among the row's threads
@@ -135,7 +139,9 @@ struct RowPos {
 };
 
 __device__ __forceinline__ RowPos row_pos(int tpr) {
-  return RowPos{(int64_t)blockIdx.x * (blockDim.x / tpr) + threadIdx.x / tpr, (int)(threadIdx.x % tpr), tpr};
+  if (tpr > kWave) return RowPos{(int64_t)blockIdx.x, (int)threadIdx.x, tpr};
+  const int sh = 31 - __builtin_clz(tpr);
+  return RowPos{(int64_t)blockIdx.x * (blockDim.x >> sh) + (threadIdx.x >> sh), (int)(threadIdx.x & (tpr - 1)), tpr};
 }
 
 // Sum / max over all threads of a row: xor butterflies within the row's lane
@@ -165,16 +171,14 @@ __device__ __forceinline__ float row_max_all(float v, float* slot, int tpr) {
   return v;
 }
 
-// Streaming access for rows longer than the register cache: chunk c of a row
-// is the c-th run of 64 * EPV columns.
+// Streaming access for rows longer than the register cache: EPV columns from
+// `col` on.
 template <typename T, int EPV>
 __device__ __forceinline__ void load_chunk(const T* __restrict__ p, int64_t n, int64_t col,
                                            float (&v)[EPV], float fill) {
-  if constexpr (EPV > 1) {
-    if (col + EPV <= n) {
-      Elem<T>::unpack(*reinterpret_cast<const uint4*>(p + col), v);
-      return;
-    }
+  if (col + EPV <= n) {
+    Elem<T>::unpack(load16(p + col), v);
+    return;
   }
 #pragma unroll
   for (int e = 0; e < EPV; ++e) v[e] = (col + e < n) ? Elem<T>::load(p + col + e) : fill;
@@ -183,48 +187,35 @@ __device__ __forceinline__ void load_chunk(const T* __restrict__ p, int64_t n, i
 template <typename T, int EPV>
 __device__ __forceinline__ void store_chunk(T* __restrict__ p, int64_t n, int64_t col,
                                             const float (&v)[EPV]) {
-  if constexpr (EPV > 1) {
-    if (col + EPV <= n) {
-      store16_stream(p + col, Elem<T>::pack(v));
-      return;
-    }
+  if (col + EPV <= n) {
+    store16_row(p + col, Elem<T>::pack(v));
+    return;
   }
 #pragma unroll
   for (int e = 0; e < EPV; ++e)
     if (col + e < n) Elem<T>::store(p + col + e, v[e]);
 }
 
-// EPV consecutive f32 values (zero past n), as 16-byte loads where they fit.
-template <int EPV>
-__device__ __forceinline__ void load_f32_run(const float* __restrict__ p, int64_t n,
-                                             int64_t col, float (&u)[EPV]) {
-  if constexpr (EPV % 4 == 0) {
-    if (col + EPV <= n) {
-#pragma unroll
-      for (int q = 0; q < EPV / 4; ++q)
-        Elem<float>::unpack(*reinterpret_cast<const uint4*>(p + col + 4 * q), &u[4 * q]);
-      return;
-    }
-  }
-#pragma unroll
-  for (int e = 0; e < EPV; ++e) u[e] = (col + e < n) ? p[col + e] : 0.f;
-}
-
 // EPV consecutive values of a per-column vector of storage type W (f32 or
-// bf16 bits) as f32, with 16-byte loads when `vec` (16-byte aligned base) and
-// the run is whole; zero past n.
+// bf16 bits) as f32, in 16-byte loads (8-byte where EPV bf16 values fill no
+// more) where the run is whole; zero past n.
 template <typename W, int EPV>
-__device__ __forceinline__ void load_vec_run(const W* __restrict__ p, int64_t n, int64_t col,
-                                             bool vec, float (&u)[EPV]) {
-  constexpr int BYTES = EPV * (int)sizeof(W);
+__device__ __forceinline__ void load_vec_run(const W* __restrict__ p, int64_t n, int64_t col, float (&u)[EPV]) {
   constexpr int PER16 = 16 / (int)sizeof(W);
-  if constexpr (BYTES % 16 == 0) {
-    if (vec && col + EPV <= n) {
-      const uint4* q = reinterpret_cast<const uint4*>(p + col);
+  if (col + EPV <= n) {
+    if constexpr (EPV % PER16 == 0) {
 #pragma unroll
-      for (int i = 0; i < BYTES / 16; ++i) Elem<W>::unpack(q[i], &u[i * PER16]);
-      return;
+      for (int i = 0; i < EPV / PER16; ++i) Elem<W>::unpack(load16(p + col + i * PER16), &u[i * PER16]);
+    } else {
+      static_assert(EPV == 4 && sizeof(W) == 2, "half a vector of bf16");
+      typedef uint32_t half_t __attribute__((ext_vector_type(2), aligned(2)));
+      const half_t h = *reinterpret_cast<const half_t*>(p + col);
+      u[0] = __uint_as_float(h[0] << 16);
+      u[1] = __uint_as_float(h[0] & 0xffff0000u);
+      u[2] = __uint_as_float(h[1] << 16);
+      u[3] = __uint_as_float(h[1] & 0xffff0000u);
     }
+    return;
   }
 #pragma unroll
   for (int e = 0; e < EPV; ++e) u[e] = (col + e < n) ? Elem<W>::load(p + col + e) : 0.f;
@@ -234,19 +225,18 @@ __device__ __forceinline__ int64_t unit_index() {
   return (int64_t)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
 }
 
-// `fill` for a null vector, else EPV consecutive values from index i (a
-// multiple of EPV) of a 16-byte aligned f32 or bf16 vector, with 16-byte loads
-// where the run fills them.
+// `fill` for a null vector, else the EPV values from index i of an f32 or
+// bf16 vector of n values (zero past n).
 template <int EPV>
-__device__ __forceinline__ void load_vec_any(const void* p, int dtype, int64_t i, float (&out)[EPV],
+__device__ __forceinline__ void load_vec_any(const void* p, int dtype, int64_t n, int64_t i, float (&out)[EPV],
                                              float fill) {
   if (!p) {
 #pragma unroll
     for (int e = 0; e < EPV; ++e) out[e] = fill;
   } else if (dtype == HMX_DTYPE_F32) {
-    load_vec_run<float, EPV>((const float*)p, i + EPV, i, true, out);
+    load_vec_run<float, EPV>((const float*)p, n, i, out);
   } else {
-    load_vec_run<uint16_t, EPV>((const uint16_t*)p, i + EPV, i, true, out);
+    load_vec_run<uint16_t, EPV>((const uint16_t*)p, n, i, out);
   }
 }
 
@@ -302,12 +292,7 @@ __device__ __forceinline__ void load_row_raw(const T* __restrict__ p, int li, in
 #pragma unroll
   for (int j = 0; j < VPL; ++j) {
     const T* q = p + ((int64_t)j * tpr + li) * EPV;
-    if constexpr (std::is_same_v<T, float>) {
-      const u32x4_t nt = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(q));
-      raw[j] = make_uint4(nt[0], nt[1], nt[2], nt[3]);
-    } else {
-      raw[j] = *reinterpret_cast<const uint4*>(q);
-    }
+    raw[j] = std::is_same_v<T, float> ? load16_nt(q) : load16(q);
   }
 }
 
@@ -345,14 +330,14 @@ __device__ __forceinline__ void group_norm_rows_body(const T* x, T* y, const Gro
   for (int j = 0; j < VPL; ++j) {
     const int64_t col0 = col_of<EPV>(j, li, tpr, 0);
     float t[EPV];
-    load_vec_any<EPV>(a.w, a.vec_dtype, col0, t, 1.f);
+    load_vec_any<EPV>(a.w, a.vec_dtype, col0 + EPV, col0, t, 1.f);
 #pragma unroll
     for (int e = 0; e < EPV; ++e) wv[j * EPV + e] = t[e];
-    load_vec_any<EPV>(a.b, a.vec_dtype, col0, t, 0.f);
+    load_vec_any<EPV>(a.b, a.vec_dtype, col0 + EPV, col0, t, 0.f);
 #pragma unroll
     for (int e = 0; e < EPV; ++e) bv[j * EPV + e] = t[e];
     if constexpr (EXTRA) {
-      load_vec_any<EPV>(a.extra, a.vec_dtype, col0, t, 0.f);
+      load_vec_any<EPV>(a.extra, a.vec_dtype, col0 + EPV, col0, t, 0.f);
 #pragma unroll
       for (int e = 0; e < EPV; ++e) ev[j * EPV + e] = t[e];
     }
@@ -438,7 +423,7 @@ __device__ __forceinline__ void group_norm_rows_body(const T* x, T* y, const Gro
     } else {
       group_norm_finish<VPL * EPV, false>(a, v, ex);
     }
-    store_row<T, EPV, VPL, true>(y + row * n, n, li, tpr, v);
+    store_row<T, EPV, VPL, true>(y + row * n, (int)n, li, tpr, v);
     if (next >= rows) break;
     row = next;
 #pragma unroll
