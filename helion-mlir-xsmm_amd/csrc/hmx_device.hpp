@@ -49,12 +49,25 @@ __device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
 
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
+// 16 bytes at an address that keeps only its element type's alignment: gfx950
+// takes 16-byte global accesses at any element address, and only the pieces
+// that cross a cache line cost a second request.
+typedef uint32_t u32x4_any_t __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ uint4 load16(const void* p) {
+  const u32x4_any_t v = *reinterpret_cast<const u32x4_any_t*>(p);
+  return make_uint4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ uint4 load16_nt(const void* p) {
+  const u32x4_any_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any_t*>(p));
+  return make_uint4(v[0], v[1], v[2], v[3]);
+}
+
 // 16-byte store with the non-temporal (streaming) hint. Streaming kernels
 // write each output once and never read it back: with the hint the writes
 // reach HBM without allocating cache lines, which measures ~25% more write
 // bandwidth than plain stores on gfx950.
 __device__ __forceinline__ void store16_stream(void* p, const uint4& v) {
-  __builtin_nontemporal_store(u32x4_t{v.x, v.y, v.z, v.w}, (u32x4_t*)p);
+  __builtin_nontemporal_store(u32x4_any_t{v.x, v.y, v.z, v.w}, reinterpret_cast<u32x4_any_t*>(p));
 }
 
 // A 16-byte store written through to memory (the system-scope coherence bits

@@ -77,15 +77,20 @@ struct Plan {
   int splits;
   int64_t k_chunk;
   int64_t workspace_bytes;
-  // Row-major bf16 B is first transposed to [N, K] in the workspace (at
-  // offset 0, bt_bytes long) when enough output rows reuse it: the K-contiguous
-  // kernel path then reads it without register transposes.
+  // Room in the workspace (at offset 0, bt_bytes long) for a row-major bf16 B
+  // transposed to [N, K], which the launch uses where the direct-to-LDS kernels
+  // cannot read B in place and enough output rows reuse it.
   bool transpose_b;
+  // bf16 B whose rows keep no 4-byte alignment (K of [N, K], N of [K, N] odd) is
+  // first copied there with its rows padded to a multiple of 8.
+  bool pad_b;
   int64_t bt_bytes;
   // bf16 A stored [K, M] is first transposed to [M, K] in the workspace
-  // (after the transposed B, at_bytes long), and the product is planned and
-  // run as one of row-major A.
+  // (after the prepared B, at_bytes long), and the product is planned and
+  // run as one of row-major A; a row-major A of odd K is copied there with
+  // its rows padded.
   bool transpose_a;
+  bool pad_a;
   int64_t at_bytes;
   // M <= 64 against B [N, K]: the skinny kernel (tile 32 x 32 x 64, no
   // split, no workspace).
@@ -140,7 +145,7 @@ int auto_splits(TileChoice tile, int64_t tiles, int64_t m, int64_t n, int64_t k,
     const int64_t need = (int64_t)s2 * batch * m * n * 4;
     // The f32 partials' traffic (written once, read once) at most an eighth
     // of the operands'. With `fill`, bf16 128 x 128 tiles of products of at
-    // least 2^30 multiply-adds, K in whole stages, also split while the grid
+    // least 2^30 multiply-adds (rows the direct-to-LDS kernels read) also split while the grid
     // stays within one workgroup per CU, each chunk keeps 16 or more stages
     // and the partials move at most the operands' bytes: a grid of one such
     // workgroup per CU on a few CUs is latency-bound, and filling the CUs
@@ -149,7 +154,7 @@ int auto_splits(TileChoice tile, int64_t tiles, int64_t m, int64_t n, int64_t k,
     // 33.7 -> 27.9 us, 768 x 768 x 3072 24.5 -> 20.5 us; a grid past one
     // workgroup per CU loses the four-stage ring: 256 x 11008 x 4096
     // 36 -> 44.5 us in two).
-    const bool fills = fill && esz == 2 && tile.bm == 128 && k % tile.bk == 0 && kt / s2 >= 16 && tiles * s2 <= cus &&
+    const bool fills = fill && esz == 2 && tile.bm == 128 && kt / s2 >= 16 && tiles * s2 <= cus &&
                        (double)batch * m * n * k >= 1073741824.0 && need <= operand_bytes;
     if ((max_ws >= 0 && need > max_ws) || (2 * need > operand_bytes / 4 && !fills)) break;
     splits = s2;
@@ -214,7 +219,7 @@ int make_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int64_t batch, int 
     plan.tile = kSkinny;
     plan.splits = 1;
     plan.k_chunk = k;
-    plan.transpose_b = plan.transpose_a = false;
+    plan.transpose_b = plan.transpose_a = plan.pad_a = plan.pad_b = false;
     plan.bt_bytes = plan.at_bytes = 0;
     plan.workspace_bytes = 0;
     return HMX_OK;
@@ -228,20 +233,32 @@ int make_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int64_t batch, int 
   // x 4096 203 -> 55, 4096 x 1000 x 4096 105 -> 62), except for whole 256 x
   // 256 tiles the in-place kernel takes with N up to 4096, where the two
   // measure level (4096^3: 120 us transposed).
+  const int64_t k8 = ceil_div(k, 8) * 8;
+  const int64_t b_elems = b_layout == HMX_B_TRANS ? n * k8 : k * (ceil_div(n, 8) * 8);
   const bool ta_in_place = m % 256 == 0 && n % 256 == 0 && k % 64 == 0 && (m / 256) * (n / 256) >= cus &&
                            n <= 4096;
   plan.transpose_a = bf16 && trans_a && !program && batch == 1 && transpose_a_enabled() &&
                      (b_layout == HMX_B_ROW || b_layout == HMX_B_TRANS) && m >= kTransposeAMin &&
-                     n >= kTransposeAMin && k >= kTransposeAMin && m * k * 2 < INT32_MAX && !ta_in_place;
-  plan.at_bytes = plan.transpose_a ? ceil_div(m * k * 2, 256) * 256 : 0;
-  if (plan.transpose_a && max_ws >= 0 && plan.at_bytes > max_ws) {
-    plan.transpose_a = false;
-    plan.at_bytes = 0;
+                     n >= kTransposeAMin && k >= kTransposeAMin && m * k8 * 2 < INT32_MAX && !ta_in_place;
+  // Rows that keep no 4-byte alignment (odd K or N): the direct-to-LDS kernels
+  // cannot read them, and the register-staged kernel is slower at every size
+  // by more than the copy takes, so each such operand is copied once with its
+  // rows padded (one launch for both; a zero K tail). In place (element by
+  // element; in 16-byte loads) -> copied: 4000 x 4000 x 4001 1264, - -> 112 us,
+  // 200 x 4096 x 4095 with B [N, K] 496, 113 -> 36, 100 x 11008 x 4095 with it
+  // 283, 75 -> 56, 64 x 64 x 501 46, 38 -> 11.
+  const bool pads = bf16 && (b_layout == HMX_B_ROW || b_layout == HMX_B_TRANS) && k >= 63 &&
+                    (!trans_a || plan.transpose_a);
+  plan.pad_a = pads && !trans_a && k % 2 != 0 && m * k8 * 2 < INT32_MAX;
+  plan.pad_b = pads && (b_layout == HMX_B_TRANS ? k % 2 != 0 : n % 2 != 0) && b_elems * 2 < INT32_MAX;
+  plan.at_bytes = plan.transpose_a || plan.pad_a ? ceil_div(batch * m * k8 * 2, 256) * 256 : 0;
+  plan.bt_bytes = plan.pad_b ? ceil_div(batch * b_elems * 2, 256) * 256 : 0;
+  if (max_ws >= 0 && plan.at_bytes + plan.bt_bytes > max_ws) {
+    plan.transpose_a = plan.pad_a = plan.pad_b = false;
+    plan.at_bytes = plan.bt_bytes = 0;
   }
-  if (plan.transpose_a) {
-    trans_a = 0;
-    if (max_ws >= 0) max_ws -= plan.at_bytes;
-  }
+  if (plan.transpose_a) trans_a = 0;
+  if (max_ws >= 0) max_ws -= plan.at_bytes + plan.bt_bytes;
   const TileChoice* table = bf16 ? kBf16Tiles : kF32Tiles;
   const int count = bf16 ? (int)(sizeof(kBf16Tiles) / sizeof(TileChoice))
                          : (int)(sizeof(kF32Tiles) / sizeof(TileChoice));
@@ -297,7 +314,9 @@ int make_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int64_t batch, int 
   const int64_t tiles = ceil_div(m, plan.tile.bm) * ceil_div(n, plan.tile.bn) * batch;
   const int64_t kt = ceil_div(k, plan.tile.bk);
   if (splits == 0) {
-    splits = auto_splits(plan.tile, tiles, m, n, k, batch, bf16 ? 2 : 4, max_ws, cus, true);
+    // (Rows read at 16-byte alignment: their own, or the padded copies'.)
+    const bool fill = bf16 && !trans_a && (k % 8 == 0 || plan.transpose_a || plan.pad_a);
+    splits = auto_splits(plan.tile, tiles, m, n, k, batch, bf16 ? 2 : 4, max_ws, cus, fill);
     if (!bf16 && plan.tile.bm < 256 && tiles * 4 <= cus)
       splits = std::max(splits, small_f32_splits(tiles, kt, batch * m * n, max_ws, cus));
   }
@@ -321,21 +340,18 @@ int make_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int64_t batch, int 
       splits > 1 || (program && !program_fused_shape(plan, bf16, m, n, k, trans_a, b_layout))
           ? (int64_t)std::max(splits, 1) * batch * m * n * 4
           : 0;
-  plan.bt_bytes = ceil_div(n * k * 2, 256) * 256;
-  // The direct-to-LDS kernels read row-major B in place (256 x 256 tiles,
-  // ragged M and N too, or transposed A on whole tiles; 128 x 128 tiles of
-  // row-major A) when K chunks are whole 64-element stages; other bf16 shapes
-  // with enough rows read it transposed up front.
-  // (N % 8 == 0: the rows of a contiguous B keep the 16-byte alignment those
-  // loads need.)
+  // The direct-to-LDS kernels read row-major B in place where its rows keep
+  // their alignment; K in whole stages and N a multiple of 8 always do. Other
+  // bf16 shapes with enough rows get room to transpose it up front, for the
+  // launches that take another kernel.
   const bool dma_reads_b = k % 64 == 0 && plan.k_chunk % 64 == 0 && n % 8 == 0 &&
                            ((plan.tile.bm == 256 && (!trans_a || (m % 256 == 0 && n % 256 == 0))) ||
                             (plan.tile.bm == 128 && !trans_a));
-  plan.transpose_b = bf16 && b_layout == HMX_B_ROW && !dma_reads_b && batch == 1 &&
-                     m >= kTransposeMinRows &&
-                     n * k * 2 < INT32_MAX &&
-                     (max_ws < 0 || plan.bt_bytes + partial_bytes <= max_ws);
-  if (!plan.transpose_b) plan.bt_bytes = 0;
+  const int64_t bt = ceil_div(n * k * 2, 256) * 256;
+  plan.transpose_b = bf16 && b_layout == HMX_B_ROW && !dma_reads_b && !plan.pad_b && batch == 1 &&
+                     m >= kTransposeMinRows && n * k * 2 < INT32_MAX &&
+                     (max_ws < 0 || bt + partial_bytes <= max_ws);
+  if (plan.transpose_b) plan.bt_bytes = bt;
   plan.workspace_bytes = plan.bt_bytes + plan.at_bytes + partial_bytes;
   return HMX_OK;
 }
@@ -368,16 +384,14 @@ int64_t whole_round_columns(int64_t tiles_m, int64_t tiles_n, int cus) {
   return (tiles - tail) / tiles_m;
 }
 
-// The direct-to-LDS kernels finish C from registers for identity, ReLU and
-// SiLU, which store bf16 C as 4-byte aligned column pairs; every other
+// The 32x32 direct-to-LDS kernels finish C from registers for identity, ReLU
+// and SiLU, which store bf16 C as 4-byte aligned column pairs (the 16x16x32
+// kernel stores 16-byte runs at any alignment); every other
 // activation and epilogue programs go through their LDS-staged epilogue,
 // which takes any alignment.
 bool dma_direct_ok(const GemmArgs& g) {
   const bool direct = g.act == HMX_EPI_IDENTITY || g.act == HMX_EPI_RELU || g.act == HMX_EPI_SILU;
-  const bool pair_ok = g.c_dtype != HMX_DTYPE_BF16 ||
-                       (g.ldc % 2 == 0 && g.stride_c % 2 == 0 && g.stride_split % 2 == 0 &&
-                        (((uintptr_t)g.c) & 3) == 0);
-  return (!direct || pair_ok) && g.k_chunk % 32 == 0 && g.k > 0;
+  return (!direct || dma_pairs_ok(g)) && g.k > 0;
 }
 
 // The kernel families a launch can take.
@@ -398,18 +412,26 @@ Kernel select_kernel(const GemmArgs& g, const Plan& plan, int ab_dtype, int la, 
                      bool bytes_ok) {
   const bool aligned = g.a.vec && g.b.vec && bytes_ok;
   const bool plain_b = lb == L_KCONTIG || lb == L_RCONTIG;
+  // The direct-to-LDS loads take 16-byte pieces at any 4-byte alignment.
+  const bool words = (g.a.vec || g.a.word) && (g.b.vec || (plain_b && g.b.word)) && bytes_ok;
   if (plan.skinny) return aligned && dma_enabled() ? Kernel::SKINNY : Kernel::SKINNY_TILES;
   if (ab_dtype == HMX_DTYPE_BF16) {
     const TileChoice t = plan.tile;
     const bool k64 = g.k % 64 == 0 && plan.k_chunk % 64 == 0;
-    // Whole 256 x 256 tiles, or ragged M and N with K chunks of whole
-    // 64-element stages and B K-contiguous or row-major.
-    const bool dma_shape = aligned && (whole || (plain_b && k64));
-    const bool ok = dma_direct_ok(g) && dma_enabled();
+    // K chunks that are not whole 64-element stages: the 16x16x32 kernel
+    // zeroes the tail, from one stage on. Epilogue programs keep the staged
+    // path there.
+    const bool mi16 = gemm_bf16_tails_ok(g);
+    const bool k_ok = k64 || (mi16 && plain_b && la == L_KCONTIG && g.k >= 63 && g.act != HMX_EPI_PROGRAM);
+    // Whole 256 x 256 tiles, or ragged M, N and K with B K-contiguous or
+    // row-major.
+    const bool dma_shape = words && k_ok && (whole || plain_b);
+    const bool ok = (dma_direct_ok(g) || (mi16 && g.k > 0)) && dma_enabled();
     if (t.bm == 256 && dma_shape && la == L_KCONTIG && (plain_b || gemm_bf16_dma_packed_ok(g, lb)) && ok)
       return Kernel::DMA;
-    if (t.bm == 256 && la == L_RCONTIG && whole && aligned && plain_b && ok) return Kernel::DMA_TA;
-    if (t.bm == 128 && la == L_KCONTIG && plain_b && aligned && k64 && ok) return Kernel::DMA128;
+    if (t.bm == 256 && la == L_RCONTIG && whole && aligned && plain_b && dma_direct_ok(g) && dma_enabled())
+      return Kernel::DMA_TA;
+    if (t.bm == 128 && dma_shape && la == L_KCONTIG && plain_b && ok) return Kernel::DMA128;
     return Kernel::BF16;
   }
   const bool guard = !(whole && aligned);
@@ -488,7 +510,7 @@ int gemm_impl(int ab_dtype, int c_dtype, const void* a, int64_t lda, int trans_a
   // front, an epilogue program and the allocation-free entry point keep the
   // register-staged kernel.
   if (!use_scratch && !program_epi && batch == 1 && !packed && !trans_a && plan.splits <= 1 &&
-      !plan.transpose_b && !plan.transpose_a && k > 0) {
+      !plan.transpose_b && !plan.transpose_a && !plan.pad_a && !plan.pad_b && k > 0) {
     const int64_t esz = dtype_bytes(ab_dtype), cb = dtype_bytes(c_dtype);
     // Rows of leading dimension ld whose span ((rows - 1) ld + k) esz stays
     // below 2^31 bytes, in whole 256-row tiles (0: not even one tile).
@@ -523,28 +545,30 @@ int gemm_impl(int ab_dtype, int c_dtype, const void* a, int64_t lda, int trans_a
       return HMX_OK;
     }
   }
-  // Workspace is checked once the launch is known (below): a B transposed up
-  // front (plan.bt_bytes), then an A transposed up front (plan.at_bytes), then
+  // Workspace is checked once the launch is known (below): a B transposed or
+  // padded up front (plan.bt_bytes), then an A (plan.at_bytes), then
   // f32 partials for split-K or a staged epilogue program. The transposed
   // operands are read K-contiguous from the workspace.
-  if (use_scratch && (plan.transpose_b || plan.transpose_a)) {
+  if (use_scratch && plan.bt_bytes + plan.at_bytes > 0) {
     const int st = scratch_of_current_device(&workspace);
     if (st != HMX_OK) return st;
     workspace_bytes = kScratchBytes;
   }
   const void* b_given = b;
-  const int64_t ldb_given = ldb;
+  const int64_t ldb_given = ldb, stride_b_given = stride_b;
   int lb_run = lb;
-  if (plan.transpose_b) {
+  const int64_t k8 = ceil_div(k, 8) * 8, n8 = ceil_div(n, 8) * 8;
+  if (plan.pad_b) {
     b = workspace;
-    ldb = k;
-    lb_run = L_KCONTIG;
+    ldb = lb == L_KCONTIG ? k8 : n8;
+    stride_b = (lb == L_KCONTIG ? n : k) * ldb;
   }
   const void* a_given = a;
-  const int64_t lda_given = lda;
-  if (plan.transpose_a) {
+  const int64_t lda_given = lda, stride_a_given = stride_a;
+  if (plan.transpose_a || plan.pad_a) {
     a = workspace ? (const char*)workspace + plan.bt_bytes : nullptr;
-    lda = k;
+    lda = k8;
+    stride_a = m * lda;
     trans_a = 0;
   }
   int64_t tiles_m = ceil_div(m, plan.tile.bm), tiles_n = ceil_div(n, plan.tile.bn);
@@ -555,23 +579,38 @@ int gemm_impl(int ab_dtype, int c_dtype, const void* a, int64_t lda, int trans_a
   const int64_t vec_elems = 16 / esz;
   GemmArgs g{};
   const int la = trans_a ? L_RCONTIG : L_KCONTIG;
+  // 4-byte aligned rows (f32 always).
+  auto words_of = [&](const void* p, int64_t ld, int64_t stride) {
+    return (((uintptr_t)p) & 3) == 0 && ld * esz % 4 == 0 && (batch == 1 || stride * esz % 4 == 0);
+  };
   g.a = Operand{a, lda, m, 0, 0,
-                aligned16(a) && lda % vec_elems == 0 && (batch == 1 || stride_a % vec_elems == 0), 0};
+                aligned16(a) && lda % vec_elems == 0 && (batch == 1 || stride_a % vec_elems == 0),
+                words_of(a, lda, stride_a), 0};
   const int64_t b_rows = packed ? (lb == L_BLOCKED_VNNI || lb == L_BLOCKED ? ceil_div(n, 32) * 32
                                                                            : ceil_div(n, b_panel) * b_panel)
                                 : n;
-  g.b = Operand{b, ldb, b_rows, b_panel, b_kpad,
-                aligned16(b) && (packed || ldb % vec_elems == 0) &&
-                    (batch == 1 || stride_b % vec_elems == 0),
-                0};
   // Bytes spanned by one batch slice of each operand: the buffer-load
-  // range of the whole-tile path, which needs it below 2^31.
-  const int64_t a_bytes = (trans_a ? (k - 1) * lda + m : (m - 1) * lda + k) * esz;
-  const int64_t b_bytes =
-      packed ? b_rows * b_kpad * esz : (lb_run == L_RCONTIG ? (k - 1) * ldb + n : (n - 1) * ldb + k) * esz;
-  const bool bytes_ok = a_bytes < INT32_MAX && b_bytes < INT32_MAX;
-  g.a.bytes = bytes_ok ? (int32_t)a_bytes : 0;
-  g.b.bytes = bytes_ok ? (int32_t)b_bytes : 0;
+  // range of the direct-to-LDS and whole-tile paths, which needs it below
+  // 2^31. The range is checked by 4-byte words: an odd count of bf16 elements
+  // keeps its last word (the word holds an element, so it lies in the
+  // allocation).
+  auto words = [](int64_t bytes) { return (int32_t)((bytes + 3) & ~(int64_t)3); };
+  const bool prepared_a = plan.transpose_a || plan.pad_a;
+  const int64_t a_bytes = (prepared_a ? m * lda : trans_a ? (k - 1) * lda + m : (m - 1) * lda + k) * esz;
+  bool bytes_ok = false;
+  auto bind_b = [&]() {
+    g.b = Operand{b, ldb, b_rows, b_panel, b_kpad,
+                  aligned16(b) && (packed || ldb % vec_elems == 0) && (batch == 1 || stride_b % vec_elems == 0),
+                  words_of(b, packed ? 0 : ldb, stride_b), 0};
+    const int64_t b_bytes =
+        packed ? b_rows * b_kpad * esz
+               : (plan.pad_b ? (lb_run == L_RCONTIG ? k : n) * ldb
+                             : lb_run == L_RCONTIG ? (k - 1) * ldb + n : (n - 1) * ldb + k) * esz;
+    bytes_ok = a_bytes < INT32_MAX - 3 && b_bytes < INT32_MAX - 3;
+    g.a.bytes = bytes_ok ? words(a_bytes) : 0;
+    g.b.bytes = bytes_ok ? words(b_bytes) : 0;
+  };
+  bind_b();
   // Packed layouts read zeros (their padding) past N up to the padded extent;
   // columns past N are never stored.
   g.stride_a = stride_a;
@@ -601,6 +640,15 @@ int gemm_impl(int ab_dtype, int c_dtype, const void* a, int64_t lda, int trans_a
                plan.k_chunk % plan.tile.bk == 0 && k % plan.tile.bk == 0;
   bool guard = !(whole && g.a.vec && g.b.vec && bytes_ok);
   Kernel kind = select_kernel(g, plan, ab_dtype, la, lb_run, whole, bytes_ok);
+  const bool transpose_b = plan.transpose_b && kind == Kernel::BF16;
+  if (transpose_b) {
+    b = workspace;
+    ldb = k;
+    lb_run = L_KCONTIG;
+    bind_b();
+    guard = !(whole && g.a.vec && g.b.vec && bytes_ok);
+    kind = select_kernel(g, plan, ab_dtype, la, lb_run, whole, bytes_ok);
+  }
   if (kind == Kernel::F32 && plan.tile.bm == 256 && plan.splits < 2) {
     // The unsplit 256 x 256 f32 tile runs on the direct-to-LDS kernel only
     // (aligned operands, an epilogue it finishes): otherwise the 128 x 128
@@ -626,7 +674,7 @@ int gemm_impl(int ab_dtype, int c_dtype, const void* a, int64_t lda, int trans_a
       plan.bt_bytes + plan.at_bytes + (staged ? (int64_t)std::max(plan.splits, 1) * batch * m * n * 4 : 0);
   const char* what = plan.splits > 1 ? "split-K"
                      : staged        ? "an epilogue program on these operands"
-                                     : "the operand transpose";
+                                     : "the operands' transpose or copy";
   if (use_scratch && need > 0) {
     HMX_REQUIRE(need <= kScratchBytes,
                 "gemm_noalloc: %s needs %lld bytes of workspace and the library's scratch holds %lld%s", what,
@@ -644,14 +692,24 @@ int gemm_impl(int ab_dtype, int c_dtype, const void* a, int64_t lda, int trans_a
   void* partials = workspace ? (char*)workspace + plan.bt_bytes + plan.at_bytes : nullptr;
   if (plan.transpose_a) {
     // A [K, M] -> [M, K] in the workspace, after the transposed B.
-    launch_transpose16(a_given, (char*)workspace + plan.bt_bytes, k, m, lda_given, (hipStream_t)stream);
+    launch_transpose16(a_given, (char*)workspace + plan.bt_bytes, k, m, lda_given, k8, (hipStream_t)stream);
     const int st = check_launch("gemm A transpose");
     if (st != HMX_OK) return st;
   }
-  if (plan.transpose_b) {
+  if (transpose_b) {
     // B [K, N] -> B^T [N, K] in the workspace; the GEMM then reads it K-contiguous.
-    launch_transpose16(b_given, workspace, k, n, ldb_given, (hipStream_t)stream);
+    launch_transpose16(b_given, workspace, k, n, ldb_given, k, (hipStream_t)stream);
     const int st = check_launch("gemm B transpose");
+    if (st != HMX_OK) return st;
+  }
+  if (plan.pad_a || plan.pad_b) {
+    const bool kc = lb == L_KCONTIG;
+    const PadRows16 pa{a_given, (char*)workspace + plan.bt_bytes, plan.pad_a ? batch : 0, stride_a_given,
+                       m, k, lda_given, k8};
+    const PadRows16 pb{b_given, workspace, plan.pad_b ? batch : 0, stride_b_given,
+                       kc ? n : k, kc ? k : n, ldb_given, kc ? k8 : n8};
+    launch_pad_rows16(pa, pb, (hipStream_t)stream);
+    const int st = check_launch("gemm operand padding");
     if (st != HMX_OK) return st;
   }
   if (staged) {
@@ -667,7 +725,7 @@ int gemm_impl(int ab_dtype, int c_dtype, const void* a, int64_t lda, int trans_a
       const char* e = getenv("HMX_GEMM_STAGGER");
       return !(e && e[0] == '0');
     }();
-    g.k_stagger = stagger && plan.splits > 1 && tiles_m * tiles_n == 1;
+    g.k_stagger = stagger && plan.splits > 1 && tiles_m * tiles_n == 1 && k % 64 == 0;
     g.c = partials;
     g.c_dtype = HMX_DTYPE_F32;
     g.ldc = n;

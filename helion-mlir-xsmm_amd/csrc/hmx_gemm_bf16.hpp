@@ -96,8 +96,8 @@ struct Bf16Loader {
       if constexpr (KIND == 0) {
         const int64_t row = r0 + item / (BK / 8);
         const int64_t k = k0 + (item % (BK / 8)) * 8;
-        if (!GUARD || (o.vec && row < o.rows && k + 8 <= k_end))
-          r[i][0] = *(const uint4*)(p + offset_of<L>(o, row, k));
+        if (!GUARD || (row < o.rows && k + 8 <= k_end))
+          r[i][0] = load16(p + offset_of<L>(o, row, k));
         else
           r[i][0] = gather8(o, row, k, 0, 1, k_end);
       } else if constexpr (KIND == 1) {
@@ -105,8 +105,8 @@ struct Bf16Loader {
         const int64_t row = r0 + (item / (BK / 8)) * 8;
 #pragma unroll
         for (int kk = 0; kk < 8; ++kk) {
-          if (!GUARD || (o.vec && row + 8 <= o.rows && k + kk < k_end))
-            r[i][kk] = *(const uint4*)(p + offset_of<L>(o, row, k + kk));
+          if (!GUARD || (row + 8 <= o.rows && k + kk < k_end))
+            r[i][kk] = load16(p + offset_of<L>(o, row, k + kk));
           else
             r[i][kk] = gather8(o, row, k + kk, 1, 0, k_end);
         }
@@ -115,8 +115,8 @@ struct Bf16Loader {
         const int64_t row = r0 + (item / (BK / 8)) * 4;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          if (!GUARD || (o.vec && row + 4 <= o.rows && k + 2 * q + 2 <= k_end)) {
-            r[i][q] = *(const uint4*)(p + offset_of<L>(o, row, k + 2 * q));
+          if (!GUARD || (row + 4 <= o.rows && k + 2 * q + 2 <= k_end)) {
+            r[i][q] = load16(p + offset_of<L>(o, row, k + 2 * q));
           } else {
             uint32_t w[4];
 #pragma unroll

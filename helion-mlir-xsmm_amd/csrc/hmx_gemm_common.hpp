@@ -35,7 +35,8 @@ struct Operand {
   int64_t rows;    // logical extent along rows (M or N)
   int64_t panel;   // panel width (panel layouts)
   int64_t kpad;    // padded K (packed layouts)
-  bool vec;        // 16-byte loads allowed (alignment of base and lines)
+  bool vec;        // 16-byte aligned base and lines
+  bool word;       // 4-byte aligned base and lines
   int32_t bytes;   // extent of one batch slice in bytes (buffer loads; < 2^31)
 };
 
@@ -419,14 +420,38 @@ __device__ __forceinline__ void epilogue(const GemmArgs& g, float* lds, int spli
 // (packed B layouts at 256 x 256 only).
 void launch_gemm_bf16(const GemmArgs& g, int tile_bm, int la, int lb, bool guard, dim3 grid,
                       hipStream_t s);
-// hmx_gemm_dma.hip: direct-to-LDS bf16 kernels (64-wide K stages when K
-// chunks are whole 64-element stages, else 32-wide); whole 256 x 256 tiles, A
-// K-contiguous, B K-contiguous, row-major or (64-wide only) packed, identity /
-// ReLU / SiLU epilogue.
+// hmx_gemm_dma.hip: direct-to-LDS bf16 kernels, 256 x 256 tiles: A
+// K-contiguous, B K-contiguous, row-major or (whole tiles) packed, any epilogue.
+// M, N and (16x16x32 kernel) K need not be whole tiles.
 void launch_gemm_bf16_dma(const GemmArgs& g, int lb, dim3 grid, hipStream_t s);
 // The 64-wide direct-to-LDS kernel on 256 x 128 tiles (four waves, B
 // [N, K] or [K, N]): the columns past the last whole round of 256 x 256 tiles.
 void launch_gemm_bf16_dma_narrow(const GemmArgs& g, int lb, dim3 grid, hipStream_t s);
+// The 16x16x32 kernel (hmx_gemm_mi16_*.hip) on tiles of bm x bn with `stages` K
+// stages in LDS; ragged: M, N or the K chunks are not whole tiles. False
+// (nothing launched) where it does not apply: HMX_GEMM_MFMA=32, staggered K
+// walks, an epilogue that could not be compiled at run time.
+struct Mi16Tile {
+  int bm, bn, stages;
+  bool ragged;
+};
+bool gemm_mi16_ok(const GemmArgs& g);
+bool launch_mi16(const GemmArgs& g, int lb, Mi16Tile t, dim3 grid, hipStream_t s);
+bool launch_mi16_nt(const GemmArgs& g, Mi16Tile t, dim3 grid, hipStream_t s);
+bool launch_mi16_nn(const GemmArgs& g, Mi16Tile t, dim3 grid, hipStream_t s);
+bool launch_mi16_rounds(const GemmArgs& head, const GemmArgs& rest, int lb, unsigned head_blocks,
+                        unsigned rest_blocks, hipStream_t s);
+bool launch_mi16_rounds_nt(const GemmArgs& head, const GemmArgs& rest, unsigned head_blocks, unsigned rest_blocks,
+                           hipStream_t s);
+bool launch_mi16_rounds_nn(const GemmArgs& head, const GemmArgs& rest, unsigned head_blocks, unsigned rest_blocks,
+                           hipStream_t s);
+// Whether K chunks that are not whole stages, and bf16 C rows of any
+// alignment, may go to the direct-to-LDS launchers (the 16x16x32 kernel is
+// what runs them).
+bool gemm_bf16_tails_ok(const GemmArgs& g);
+// Whether bf16 C can be stored as 4-byte column pairs (the 32x32 kernels'
+// register epilogue).
+bool dma_pairs_ok(const GemmArgs& g);
 // Both in one launch where the 16x16x32 kernel runs both with a named
 // activation: workgroups 0 .. head_blocks - 1 take head's 256 x 256 tiles,
 // the rest rest's 256 x 128 tiles, so the tail's workgroups start as the last
@@ -438,8 +463,8 @@ bool launch_gemm_bf16_dma_rounds(const GemmArgs& head, const GemmArgs& rest, int
 // 256 x 256 tiles, K chunks of whole 64-element stages, B K-contiguous or
 // row-major.
 void launch_gemm_bf16_dma_ta(const GemmArgs& g, int lb, dim3 grid, hipStream_t s);
-// The 64-wide direct-to-LDS kernel on 128 x 128 tiles (four waves of 64 x 64,
-// B [N, K] or [K, N], K chunks of whole 64-element stages), whole or ragged.
+// The same on 128 x 128 tiles (four waves of 64 x 64, B [N, K] or [K, N]),
+// whole or ragged.
 void launch_gemm_bf16_dma128(const GemmArgs& g, int lb, dim3 grid, hipStream_t s);
 // Skinny products: M <= 64, row-major A, B [N, K], batch 1, K a multiple of
 // 64, operand spans below 2^31 bytes, 16-byte aligned rows; one workgroup per

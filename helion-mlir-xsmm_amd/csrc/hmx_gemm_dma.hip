@@ -1,20 +1,17 @@
-// Direct-to-LDS bf16 GEMM kernels for gfx950 (v_mfma_f32_32x32x16_bf16):
-// whole 256 x 256 tiles of row-major A and a B that is either K-contiguous
-// ([N, K]) or row-major ([K, N]). Operand tiles go from memory straight into
-// LDS (`buffer_load_dwordx4 ... lds`), with no VGPR staging and no LDS write
-// instructions. Two variants: 64-wide K stages (two stages of 64 KiB, below)
-// for K chunks of whole 64-element stages, and 32-wide K tiles (four stages
-// of 32 KiB, three in flight) otherwise.
+// Direct-to-LDS bf16 and f32 GEMM kernels for gfx950 on 32x32 MFMAs
+// (v_mfma_f32_32x32x16_bf16, v_mfma_f32_32x32x2_f32), the skinny kernel, and
+// the choice between these and the 16x16x32 kernel (hmx_gemm_mi16_*.hip).
+// Operand tiles go from memory straight into LDS (`buffer_load_dwordx4 ...
+// lds`), with no VGPR staging and no LDS write instructions.
 //
 // LDS tiles are unpadded: one such load fills 1 KiB of LDS contiguously
 // (lane l at byte 16 l), so bank conflicts are avoided by XOR-swizzling
 // 16-byte chunks instead -- the lane that fills slot c of tile row r fetches
 // global chunk c ^ swz(r).
-//  * A, and K-contiguous B: [256 rows][32 k], 64-byte rows (4 chunks),
-//    swz_k(r) = ((r >> 1) & 3) ^ ((r >> 3) & 1). A fragment read (16 bytes:
-//    row lane % 32, chunk 2 ks + lane / 32) then meets distinct banks whether
-//    LDS serves 8 or 16 lanes per cycle.
-//  * row-major B: [32 k][256 n], 512-byte rows (32 chunks),
+//  * A, and K-contiguous B: [256 rows][64 k], 128-byte rows (8 chunks),
+//    swz64(r) = (r >> 1) & 7. A fragment read (16 bytes: row lane % 32, one
+//    chunk) then meets distinct banks across 16 lanes.
+//  * row-major B: [64 k][256 n], 512-byte rows (32 chunks),
 //    swz_n(r) = ((r & 3) << 1) ^ ((r & 3) << 2). Fragments come from
 //    ds_read_b64_tr_b16, which transposes within each group of 16 lanes:
 //    lane j receives, as its element e, element j % 4 of the 8 bytes lane
@@ -31,181 +28,17 @@
 #include <cstdlib>
 
 #include "hmx_gemm_lds.hpp"
-#include "hmx_gemm_mi16.hpp"
 
 namespace hmx {
 namespace {
 
 
-// One instantiation per B orientation, register-epilogue class and C dtype:
-// a single straight-line epilogue keeps the accumulators out of scratch.
-template <int LB, int ACT, bool BF16>
-__global__ __launch_bounds__(256, 1) void gemm_bf16_dma_kernel(GemmArgs g) {
-  constexpr bool BT = LB == L_RCONTIG;             // B row-major [K, N]
-  constexpr int BM = 256, BN = 256, BK = 32, S = 4;
-  constexpr int ROWB = BK * 2;                     // bytes per K-contiguous tile row
-  constexpr int NROWB = BN * 2;                    // bytes per row-major B tile row
-  constexpr int A_BYTES = BM * ROWB;               // 16 KiB
-  constexpr int STAGE = A_BYTES + BN * BK * 2;     // 32 KiB
-  constexpr int FM = 4, FN = 4, WM = 128, WN = 128;
-  constexpr int LOADS = 8;                         // DMA instructions per wave per tile
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[S * STAGE];
-
-  int tm, tn;
-  tile_coords(g.tiles_m, g.tiles_n, g.xcds, tm, tn);
-  const int split = blockIdx.y, batch = blockIdx.z;
-  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
-  const int64_t k_begin = (int64_t)split * g.k_chunk;
-  const int64_t k_end = min(g.k, k_begin + g.k_chunk);
-  const int ktiles = (int)((k_end - k_begin) / BK);
-
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
-
-  const i32x4_t srd_a = make_srd((const uint16_t*)g.a.p + batch * g.stride_a, g.a.bytes);
-  const i32x4_t srd_b = make_srd((const uint16_t*)g.b.p + batch * g.stride_b, g.b.bytes);
-  // Wave w loads 16-row blocks 4w .. 4w + 3 of the A tile: lane l fills slot
-  // l % 4 of block row l / 4. Byte offsets below 2^31: the operands' byte
-  // ranges are.
-  const int drow = lane >> 2;
-  const int32_t voff_a = (int32_t)((drow * g.a.ld + ((lane & 3) ^ swz_k(drow)) * 8) * 2);
-  const int32_t soff_a = (int32_t)((m0 + wave * 64) * g.a.ld * 2);
-  const int32_t blk_a = (int32_t)(16 * g.a.ld * 2);
-  // B: K-contiguous as A; row-major in pairs of rows 8w + 2q, 8w + 2q + 1
-  // (q < 4), lane l filling slot l % 32 of row l / 32 of the pair.
-  int32_t voff_b0, voff_b1, soff_b, blk_b;
-  if constexpr (BT) {
-    const int r = lane >> 5, c = lane & 31;
-    voff_b0 = (int32_t)((r * g.b.ld + (c ^ swz_n(r)) * 8) * 2);      // even q
-    voff_b1 = (int32_t)((r * g.b.ld + (c ^ swz_n(r + 2)) * 8) * 2);  // odd q
-    soff_b = (int32_t)((wave * 8 * g.b.ld + n0) * 2);
-    blk_b = (int32_t)(2 * g.b.ld * 2);
-  } else {
-    voff_b0 = voff_b1 = (int32_t)((drow * g.b.ld + ((lane & 3) ^ swz_k(drow)) * 8) * 2);
-    soff_b = (int32_t)((n0 + wave * 64) * g.b.ld * 2);
-    blk_b = (int32_t)(16 * g.b.ld * 2);
-  }
-  const uint32_t lds_w = __builtin_amdgcn_readfirstlane(lds_addr(lds)) + wave * 4 * 1024;
-
-  // DMA q (< 8) of tile t: A blocks for q < 4, then B.
-  auto dma = [&](int t, int q) {
-    const int64_t k0 = k_begin + (int64_t)min(t, ktiles - 1) * BK;
-    const uint32_t st = lds_w + (uint32_t)((t % S) * STAGE);
-    if (q < 4) {
-      lds_dma16(srd_a, voff_a, soff_a + q * blk_a + (int32_t)(k0 * 2), st + q * 1024);
-    } else {
-      const int32_t kb = BT ? (int32_t)(k0 * g.b.ld * 2) : (int32_t)(k0 * 2);
-      lds_dma16(srd_b, (q & 1) ? voff_b1 : voff_b0, soff_b + (q - 4) * blk_b + kb,
-                st + A_BYTES + (q - 4) * 1024);
-    }
-  };
-
-  f32x16_t acc[FM][FN];
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-
-  // Fragment reads. A (and K-contiguous B): row lane % 32 of the fragment,
-  // chunk 2 ks + lane / 32.
-  const int frow = lane & 31, fk = lane >> 5, fswz = swz_k(frow);
-  const uint8_t* a_frag = lds + (wm * WM + frow) * ROWB;
-  const uint8_t* b_frag = lds + A_BYTES + (wn * WN + frow) * ROWB;
-  // Row-major B: lane s of 16-lane group gi addresses row 8 (gi / 2) + s / 4
-  // (+ 16 ks, + 4 for the second read) and the chunk holding columns
-  // wn * 128 + 32 j + 16 (gi % 2) + 4 (s % 4).
-  int b_tr[FN];
-  {
-    const int gi = lane >> 4, sl = lane & 15;
-    const int v = (2 * (gi & 1) + ((sl & 3) >> 1)) ^ swz_n(sl >> 2);
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-      b_tr[j] = A_BYTES + (8 * (gi >> 1) + (sl >> 2)) * NROWB + (wn * 16 + ((4 * j) ^ v)) * 16 + 8 * (sl & 1);
-  }
-  auto a_read = [&](int stage, int ks, int i) -> bf16x8_t {
-    return *(const bf16x8_t*)(a_frag + stage * STAGE + i * 32 * ROWB + ((2 * ks + fk) ^ fswz) * 16);
-  };
-  auto b_read = [&](int stage, int ks, int j) -> bf16x8_t {
-    if constexpr (BT) {
-      const uint8_t* p = lds + stage * STAGE + b_tr[j] + 16 * ks * NROWB;
-      return __builtin_shufflevector(lds_read_tr(p), lds_read_tr(p + 4 * NROWB), 0, 1, 2, 3, 4, 5, 6, 7);
-    } else {
-      return *(const bf16x8_t*)(b_frag + stage * STAGE + j * 32 * ROWB + ((2 * ks + fk) ^ fswz) * 16);
-    }
-  };
-
-  // The host launches this kernel only with at least one K tile per split.
-  bf16x8_t a0[FM], b0[FN], a1[FM], b1[FN];
-#pragma unroll
-  for (int t = 0; t < 3; ++t)
-#pragma unroll
-    for (int q = 0; q < LOADS; ++q) dma(t, q);
-  wait_vmem<2 * LOADS>();  // tile 0 landed
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < FM; ++i) a0[i] = a_read(0, 0, i);
-#pragma unroll
-  for (int j = 0; j < FN; ++j) b0[j] = b_read(0, 0, j);
-
-  for (int t = 0; t < ktiles; ++t) {
-    // Tiles t + 1 and t + 2 are in flight: wait for t + 1, then the barrier
-    // publishes it and frees stage (t + 3) % S (last read in step t - 1).
-    // The barrier carries no LDS fence: every LDS read of the freed stage
-    // was consumed by an MFMA of step t - 1 before it.
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"(LOADS) : "memory");
-    const int cur = t % S, nxt = t + 1 < ktiles ? (t + 1) % S : cur;
-    // 32 MFMA slots per step, each paired with at most one other memory
-    // operation: slots 0-7 read k-step 1's fragments, slots 8-15 issue the
-    // DMA of tile t + 3, slots 16-23 read the next tile's k-step 0 fragments
-    // (a quarter step ahead of the barrier that follows).
-#pragma unroll
-    for (int x = 0; x < 32; ++x) {
-      __builtin_amdgcn_sched_barrier(0);
-      const int f = x & 7;
-      if (x < 8) {
-        if (f < 4) a1[f] = a_read(cur, 1, f);
-        else b1[f - 4] = b_read(cur, 1, f - 4);
-      } else if (x < 16) {
-        dma(t + 3, f);
-      } else if (x < 24) {
-        if (f < 4) a0[f] = a_read(nxt, 0, f);
-        else b0[f - 4] = b_read(nxt, 0, f - 4);
-      }
-      const int idx = x & 15, i = idx >> 2, j = idx & 3;
-      if (x < 16)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0[i], b0[j], acc[i][j], 0, 0, 0);
-      else
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1[i], b1[j], acc[i][j], 0, 0, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  wait_vmem<0>();  // no load into LDS outlives the loop
-  if constexpr (staged_act(ACT)) {
-    // Any other activation or a program: through LDS, once every wave is
-    // done reading its last stage.
-    static_assert(4 * 32 * epi_pitch<WN>() * 4 <= S * STAGE, "staged epilogue fits the stages");
-    __syncthreads();
-    epilogue_staged<FM, FN, WM, WN, false, ACT == ACT_PROG>(g, (float*)lds, split, batch, m0, n0, wm, wn, wave,
-                                                             lane, acc);
-  } else {
-    epilogue_direct<FM, FN, WM, WN, false, ACT, BF16>(g, split, batch, m0, n0, wm, wn, lane, true, acc);
-  }
-}
-
 // ---------------------------------------------------------------------------
-// 64-wide K stages. The same operand handling with BK = 64 in two LDS stages
-// of 64 KiB: every K-contiguous load fetches whole 128-byte pieces of 8 rows,
-// so a cache line is requested once even when no other workgroup shares it
-// (split-K over long K streams each workgroup's own rows: with 32-wide tiles
-// each 64-byte half of a line was a separate request for the same line), and
-// a step has one barrier per 64 MFMAs.
-// K-contiguous tiles: [256 rows][64 k], 128-byte rows; 16-byte chunk c of row
-// r sits in slot c ^ swz64(r), swz64(r) = (r >> 1) & 7, so a fragment read
-// (row lane % 32, one chunk) meets distinct banks across 16 lanes. Row-major
-// B: [64 k][256 n], 512-byte rows swizzled as in the 32-wide kernel.
+// 64-wide K stages, two of 64 KiB in LDS: every K-contiguous load fetches whole
+// 128-byte pieces of 8 rows, so a cache line is requested once even when no
+// other workgroup shares it (split-K over long K streams each workgroup's own
+// rows: with 32-wide tiles each 64-byte half of a line was a separate request
+// for the same line), and a step has one barrier per 64 MFMAs.
 //
 // NW = 8 waves (the default: two per SIMD, 128 x 64 outputs each) or 4 (one
 // per SIMD, 128 x 128). Step t is four k-steps of 16, NS = FM * FN MFMA
@@ -543,30 +376,6 @@ __global__ __launch_bounds__(NW * 64, 1) void gemm_bf16_dma64_kernel(GemmArgs g)
     else
       epilogue_direct<FM, FN, WM, WN, true, ACT, BF16>(g, split, batch, m0, n0, wm, wn, lane, true, acc);
   }
-}
-
-// ---------------------------------------------------------------------------
-// The 16x16x32 kernel (body in hmx_gemm_mi16.hpp).
-template <int LB, int ACT, bool BF16, bool RAGGED = false, int BM = 256, int BN = 256, int NW = 8, int S = 2>
-__global__ __launch_bounds__(NW * 64, 1) void gemm_bf16_mi16_kernel(GemmArgs g) {
-  gemm_bf16_mi16_body<LB, ACT, BF16, RAGGED, BM, BN, NW, S>(g);
-}
-
-// A product of several rounds of 256 x 256 tiles and a tail of 256 x 128
-// tiles in one launch: workgroup b < head_blocks runs head's tile b, the
-// others rest's tile b - head_blocks (head_blocks a multiple of the XCD
-// count, so the XCD-aware tile order holds for both). Both are multi-round,
-// so C is streamed.
-template <int LB, int ACT, bool BF16>
-__global__ __launch_bounds__(512, 1) void gemm_bf16_mi16_rounds_kernel(GemmArgs head, GemmArgs rest,
-                                                                        int head_blocks) {
-  constexpr int kHead = mi16_lds_bytes<ACT, 256, 256, 8, 2>(), kTail = mi16_lds_bytes<ACT, 256, 128, 8, 2>();
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[kHead > kTail ? kHead : kTail];
-  const int b = (int)blockIdx.x;
-  if (b < head_blocks)
-    gemm_bf16_mi16_body<LB, ACT, BF16, false, 256, 256, 8, 2>(head, lds, b, false);
-  else
-    gemm_bf16_mi16_body<LB, ACT, BF16, false, 256, 128, 8, 2>(rest, lds, b - head_blocks, false);
 }
 
 // ---------------------------------------------------------------------------
@@ -925,24 +734,6 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_skinny_kernel(GemmArgs g) {
   }
 }
 
-// The 16x16x32 MFMA kernel for the eight-wave 256 x 256 tiles unless the
-// environment sets HMX_GEMM_MFMA=32 (the 32x32x16 kernel, for comparison).
-bool mfma16_enabled() {
-  static const bool on = [] {
-    const char* e = getenv("HMX_GEMM_MFMA");
-    return !(e && e[0] == '3');
-  }();
-  return on;
-}
-
-// The 16x16x32 kernel's conditions beyond its template's: no stagger, and
-// bf16 C in 16-byte row pieces.
-bool mi16_args_ok(const GemmArgs& g) {
-  const bool rows16 = g.c_dtype != HMX_DTYPE_BF16 || ((((uintptr_t)g.c) & 15) == 0 && g.ldc % 8 == 0 &&
-                                                      g.stride_c % 8 == 0 && g.stride_split % 8 == 0);
-  return !g.k_stagger && rows16 && mfma16_enabled();
-}
-
 // Eight waves (two per SIMD) unless the environment sets HMX_GEMM_WAVES=4:
 // the second wave of a SIMD issues MFMAs while the first waits at the stage
 // barrier or on an LDS read (measured: 2-5 % faster on configs 3-5).
@@ -954,91 +745,53 @@ bool eight_waves() {
   return eight;
 }
 
-template <int LB, bool BF16, bool K64, int NW = 4>
+template <int LB, bool BF16, int NW>
 void launch_bf16_dma_c(const GemmArgs& g, dim3 grid, hipStream_t s) {
-  if constexpr (K64 && NW == 8 &&
-                (LB == L_KCONTIG || LB == L_RCONTIG || LB == L_VNNI_PANELS || LB == L_PANELS || LB == L_BLOCKED)) {
-    if (mi16_args_ok(g)) {
-      switch (g.act) {
-        case HMX_EPI_IDENTITY: launch(gemm_bf16_mi16_kernel<LB, ACT_ID, BF16>, grid, 512, s, g); return;
-        case HMX_EPI_RELU: launch(gemm_bf16_mi16_kernel<LB, ACT_RELU, BF16>, grid, 512, s, g); return;
-        case HMX_EPI_SILU: launch(gemm_bf16_mi16_kernel<LB, ACT_SILU, BF16>, grid, 512, s, g); return;
-        default:
-          // Other epilogues: compiled into the register epilogue at run
-          // time; else the staged epilogue, which stores 16-byte runs of C
-          // rows (f32 C: 4-element aligned rows too).
-          if (launch_mi16_jit(g, LB, BF16, false, 256, 256, 8, 2, grid, s) == HMX_OK) return;
-          if (BF16 || ((((uintptr_t)g.c) & 15) == 0 && g.ldc % 4 == 0 && g.stride_c % 4 == 0 &&
-                       g.stride_split % 4 == 0)) {
-            if (g.act == HMX_EPI_PROGRAM) launch(gemm_bf16_mi16_kernel<LB, ACT_PROG, BF16>, grid, 512, s, g);
-            else launch(gemm_bf16_mi16_kernel<LB, ACT_ANY, BF16>, grid, 512, s, g);
-            return;
-          }
-          break;
-      }
+  if constexpr (NW == 8) {
+    if (launch_mi16(g, LB, Mi16Tile{256, 256, 2, false}, grid, s)) return;
+  }
+  if constexpr (!BF16 && NW == 8 && (LB == L_KCONTIG || LB == L_RCONTIG)) {
+    // Split-K grids of one tile per slice (k_stagger): no other workgroup
+    // reads a workgroup's operand rows, so its loads are non-temporal.
+    if (g.k_stagger && g.act == HMX_EPI_IDENTITY) {
+      launch(gemm_bf16_dma64_kernel<LB, ACT_ID, false, 8, 256, false, 256, false, true>, grid, NW * 64, s, g);
+      return;
     }
   }
-  if constexpr (K64) {
-    if constexpr (!BF16 && NW == 8 && (LB == L_KCONTIG || LB == L_RCONTIG)) {
-      // Split-K grids of one tile per slice (k_stagger): no other workgroup
-      // reads a workgroup's operand rows, so its loads are non-temporal.
-      if (g.k_stagger && g.act == HMX_EPI_IDENTITY) {
-        launch(gemm_bf16_dma64_kernel<LB, ACT_ID, false, 8, 256, false, 256, false, true>, grid, NW * 64, s, g);
-        return;
-      }
-    }
-    switch (g.act) {
-      case HMX_EPI_RELU: launch(gemm_bf16_dma64_kernel<LB, ACT_RELU, BF16, NW, 256>, grid, NW * 64, s, g); break;
-      case HMX_EPI_SILU: launch(gemm_bf16_dma64_kernel<LB, ACT_SILU, BF16, NW, 256>, grid, NW * 64, s, g); break;
-      case HMX_EPI_IDENTITY: launch(gemm_bf16_dma64_kernel<LB, ACT_ID, BF16, NW, 256>, grid, NW * 64, s, g); break;
-      default:
-        if (g.act == HMX_EPI_PROGRAM) launch(gemm_bf16_dma64_kernel<LB, ACT_PROG, BF16, NW, 256>, grid, NW * 64, s, g);
-        else launch(gemm_bf16_dma64_kernel<LB, ACT_ANY, BF16, NW, 256>, grid, NW * 64, s, g);
-        break;
-    }
-  } else if constexpr (LB != L_VNNI_PANELS) {
-    switch (g.act) {
-      case HMX_EPI_RELU: launch(gemm_bf16_dma_kernel<LB, ACT_RELU, BF16>, grid, 256, s, g); break;
-      case HMX_EPI_SILU: launch(gemm_bf16_dma_kernel<LB, ACT_SILU, BF16>, grid, 256, s, g); break;
-      case HMX_EPI_IDENTITY: launch(gemm_bf16_dma_kernel<LB, ACT_ID, BF16>, grid, 256, s, g); break;
-      default:
-        if (g.act == HMX_EPI_PROGRAM) launch(gemm_bf16_dma_kernel<LB, ACT_PROG, BF16>, grid, 256, s, g);
-        else launch(gemm_bf16_dma_kernel<LB, ACT_ANY, BF16>, grid, 256, s, g);
-        break;
-    }
+  switch (g.act) {
+    case HMX_EPI_RELU: launch(gemm_bf16_dma64_kernel<LB, ACT_RELU, BF16, NW, 256>, grid, NW * 64, s, g); break;
+    case HMX_EPI_SILU: launch(gemm_bf16_dma64_kernel<LB, ACT_SILU, BF16, NW, 256>, grid, NW * 64, s, g); break;
+    case HMX_EPI_IDENTITY: launch(gemm_bf16_dma64_kernel<LB, ACT_ID, BF16, NW, 256>, grid, NW * 64, s, g); break;
+    default:
+      if (g.act == HMX_EPI_PROGRAM) launch(gemm_bf16_dma64_kernel<LB, ACT_PROG, BF16, NW, 256>, grid, NW * 64, s, g);
+      else launch(gemm_bf16_dma64_kernel<LB, ACT_ANY, BF16, NW, 256>, grid, NW * 64, s, g);
+      break;
   }
 }
 
-template <int LB, bool K64>
+template <int LB>
 void launch_bf16_dma_b(const GemmArgs& g, dim3 grid, hipStream_t s) {
-  if (eight_waves() && K64) {
-    if (g.c_dtype == HMX_DTYPE_BF16)
-      launch_bf16_dma_c<LB, true, K64, 8>(g, grid, s);
-    else
-      launch_bf16_dma_c<LB, false, K64, 8>(g, grid, s);
-    return;
+  const bool bf16 = g.c_dtype == HMX_DTYPE_BF16;
+  if (eight_waves()) {
+    if (bf16) launch_bf16_dma_c<LB, true, 8>(g, grid, s);
+    else launch_bf16_dma_c<LB, false, 8>(g, grid, s);
+  } else {
+    if (bf16) launch_bf16_dma_c<LB, true, 4>(g, grid, s);
+    else launch_bf16_dma_c<LB, false, 4>(g, grid, s);
   }
-  if (g.c_dtype == HMX_DTYPE_BF16)
-    launch_bf16_dma_c<LB, true, K64>(g, grid, s);
-  else
-    launch_bf16_dma_c<LB, false, K64>(g, grid, s);
-}
-
-// The 64-wide kernel takes every K chunk of whole 64-element stages unless the
-// environment sets HMX_GEMM_DMA64=0 (which keeps the 32-wide kernel, for
-// comparison).
-bool dma64_enabled() {
-  static const bool on = [] {
-    const char* e = getenv("HMX_GEMM_DMA64");
-    return !(e && e[0] == '0');
-  }();
-  return on;
 }
 
 }  // namespace
 
+bool dma_pairs_ok(const GemmArgs& g) {
+  return g.c_dtype != HMX_DTYPE_BF16 ||
+         (g.ldc % 2 == 0 && g.stride_c % 2 == 0 && g.stride_split % 2 == 0 && (((uintptr_t)g.c) & 3) == 0);
+}
+
+bool gemm_bf16_tails_ok(const GemmArgs& g) { return eight_waves() && gemm_mi16_ok(g); }
+
 bool gemm_bf16_dma_packed_ok(const GemmArgs& g, int lb) {
-  if (!(g.k_chunk % 64 == 0 && g.k % 64 == 0 && dma64_enabled())) return false;
+  if (g.k_chunk % 64 != 0 || g.k % 64 != 0) return false;
   if (lb == L_PANELS) return g.b.panel % 8 == 0;
   if (lb == L_BLOCKED) return true;
   if (lb != L_VNNI_PANELS && lb != L_BLOCKED_VNNI) return false;
@@ -1050,22 +803,7 @@ template <int LB, bool BF16>
 void launch_bf16_dma_narrow(const GemmArgs& g, dim3 grid, hipStream_t s) {
   // Eight waves of 128 x 32 (two per SIMD): config 4's tail 60.5 -> 58.8 us
   // against four of 128 x 64.
-  if (mi16_args_ok(g)) {
-    switch (g.act) {
-      case HMX_EPI_IDENTITY:
-        launch(gemm_bf16_mi16_kernel<LB, ACT_ID, BF16, false, 256, 128, 8>, grid, 512, s, g);
-        return;
-      case HMX_EPI_RELU:
-        launch(gemm_bf16_mi16_kernel<LB, ACT_RELU, BF16, false, 256, 128, 8>, grid, 512, s, g);
-        return;
-      case HMX_EPI_SILU:
-        launch(gemm_bf16_mi16_kernel<LB, ACT_SILU, BF16, false, 256, 128, 8>, grid, 512, s, g);
-        return;
-      default:
-        if (launch_mi16_jit(g, LB, BF16, false, 256, 128, 8, 2, grid, s) == HMX_OK) return;
-        break;
-    }
-  }
+  if (launch_mi16(g, LB, Mi16Tile{256, 128, 2, false}, grid, s)) return;
   switch (g.act) {
     case HMX_EPI_RELU: launch(gemm_bf16_dma64_kernel<LB, ACT_RELU, BF16, 4, 128>, grid, 256, s, g); break;
     case HMX_EPI_SILU: launch(gemm_bf16_dma64_kernel<LB, ACT_SILU, BF16, 4, 128>, grid, 256, s, g); break;
@@ -1092,37 +830,11 @@ bool launch_gemm_bf16_dma_rounds(const GemmArgs& head, const GemmArgs& rest, int
   // The conditions under which launch_gemm_bf16_dma and _narrow both take the
   // 16x16x32 kernel (its prebuilt named activations, or any other epilogue
   // compiled in at run time).
-  const bool k64 = head.k_chunk % 64 == 0 && head.k % 64 == 0 && dma64_enabled();
-  const bool named = head.act == HMX_EPI_IDENTITY || head.act == HMX_EPI_RELU || head.act == HMX_EPI_SILU;
-  if (!fused_rounds_enabled() || !k64 || !eight_waves() || !mi16_args_ok(head) || !mi16_args_ok(rest) ||
-      (lb != L_KCONTIG && lb != L_RCONTIG) || head_blocks % (unsigned)std::max(head.xcds, 1) != 0 ||
-      head.m % 256 != 0 || head.n % 256 != 0)
+  const bool k64 = head.k_chunk % 64 == 0 && head.k % 64 == 0;
+  if (!fused_rounds_enabled() || !k64 || !eight_waves() || (lb != L_KCONTIG && lb != L_RCONTIG) ||
+      head_blocks % (unsigned)std::max(head.xcds, 1) != 0 || head.m % 256 != 0 || head.n % 256 != 0)
     return false;
-  // Other epilogues (programs, the other activations): the same launch with
-  // the epilogue compiled in, where run-time compilation is on.
-  if (!named)
-    return launch_mi16_rounds_jit(head, rest, lb, head.c_dtype == HMX_DTYPE_BF16, head_blocks, rest_blocks, s) ==
-           HMX_OK;
-  const dim3 grid(head_blocks + rest_blocks);
-  const int hb = (int)head_blocks;
-  auto go = [&](auto lb_c, auto bf16_c) {
-    constexpr int LBc = decltype(lb_c)::value;
-    constexpr bool BF = decltype(bf16_c)::value;
-    switch (head.act) {
-      case HMX_EPI_RELU: launch(gemm_bf16_mi16_rounds_kernel<LBc, ACT_RELU, BF>, grid, 512, s, head, rest, hb); break;
-      case HMX_EPI_SILU: launch(gemm_bf16_mi16_rounds_kernel<LBc, ACT_SILU, BF>, grid, 512, s, head, rest, hb); break;
-      default: launch(gemm_bf16_mi16_rounds_kernel<LBc, ACT_ID, BF>, grid, 512, s, head, rest, hb); break;
-    }
-  };
-  const bool bf16 = head.c_dtype == HMX_DTYPE_BF16;
-  if (lb == L_RCONTIG) {
-    if (bf16) go(std::integral_constant<int, L_RCONTIG>{}, std::true_type{});
-    else go(std::integral_constant<int, L_RCONTIG>{}, std::false_type{});
-  } else {
-    if (bf16) go(std::integral_constant<int, L_KCONTIG>{}, std::true_type{});
-    else go(std::integral_constant<int, L_KCONTIG>{}, std::false_type{});
-  }
-  return true;
+  return launch_mi16_rounds(head, rest, lb, head_blocks, rest_blocks, s);
 }
 
 void launch_gemm_bf16_dma_narrow(const GemmArgs& g, int lb, dim3 grid, hipStream_t s) {
@@ -1141,15 +853,12 @@ void launch_gemm_bf16_dma_narrow(const GemmArgs& g, int lb, dim3 grid, hipStream
 // edge rows and columns and the guarded edge epilogue.
 template <int LB, bool BF16>
 void launch_bf16_dma_ragged(const GemmArgs& g, dim3 grid, hipStream_t s) {
-  if (eight_waves() && mi16_args_ok(g)) {
-    switch (g.act) {
-      case HMX_EPI_IDENTITY: launch(gemm_bf16_mi16_kernel<LB, ACT_ID, BF16, true>, grid, 512, s, g); return;
-      case HMX_EPI_RELU: launch(gemm_bf16_mi16_kernel<LB, ACT_RELU, BF16, true>, grid, 512, s, g); return;
-      case HMX_EPI_SILU: launch(gemm_bf16_mi16_kernel<LB, ACT_SILU, BF16, true>, grid, 512, s, g); return;
-      default:
-        if (launch_mi16_jit(g, LB, BF16, true, 256, 256, 8, 2, grid, s) == HMX_OK) return;
-        break;
-    }
+  if (eight_waves() && launch_mi16(g, LB, Mi16Tile{256, 256, 2, true}, grid, s)) return;
+  if (g.k_chunk % 64 != 0 || g.k % 64 != 0 || !dma_pairs_ok(g)) {
+    // An epilogue that could not be compiled at run time, on a K tail or C
+    // rows that the kernels below do not take.
+    launch_gemm_bf16(g, 256, L_KCONTIG, LB, true, grid, s);
+    return;
   }
   switch (g.act) {
     case HMX_EPI_RELU: launch(gemm_bf16_dma64_kernel<LB, ACT_RELU, BF16, 8, 256, true>, grid, 512, s, g); break;
@@ -1176,26 +885,22 @@ int mi16_stages128(const GemmArgs& g, dim3 grid) {
   return (int64_t)grid.x * grid.y * grid.z <= g.cus ? 4 : 2;
 }
 
-template <int LB, bool BF16, bool RAGGED, int S>
-bool launch_mi16_128(const GemmArgs& g, dim3 grid, hipStream_t s) {
-  switch (g.act) {
-    case HMX_EPI_IDENTITY: launch(gemm_bf16_mi16_kernel<LB, ACT_ID, BF16, RAGGED, 128, 128, 4, S>, grid, 256, s, g); return true;
-    case HMX_EPI_RELU: launch(gemm_bf16_mi16_kernel<LB, ACT_RELU, BF16, RAGGED, 128, 128, 4, S>, grid, 256, s, g); return true;
-    case HMX_EPI_SILU: launch(gemm_bf16_mi16_kernel<LB, ACT_SILU, BF16, RAGGED, 128, 128, 4, S>, grid, 256, s, g); return true;
-    default: return false;
-  }
-}
-
 template <int LB, bool BF16, bool RAGGED>
 void launch_bf16_dma128_c(const GemmArgs& g, dim3 grid, hipStream_t s) {
   // The 16x16x32 kernel from 16 stages per split on (1000 x 4096 x 4096:
-  // 51 -> 44 us); short chunks (1024^3 split four ways: 16 -> 17.5 us) keep
-  // the 32x32x16 kernel.
-  if (mi16_args_ok(g) && g.k_chunk >= 16 * 64) {
-    const int stages = mi16_stages128(g, grid);
-    const bool done = stages == 4 ? launch_mi16_128<LB, BF16, RAGGED, 4>(g, grid, s)
-                                  : launch_mi16_128<LB, BF16, RAGGED, 2>(g, grid, s);
-    if (done || launch_mi16_jit(g, LB, BF16, RAGGED, 128, 128, 4, stages, grid, s) == HMX_OK) return;
+  // 51 -> 44 us) and for ragged tiles, whose C it stores in 16-byte runs where
+  // the 32x32x16 kernel's edge tiles go element by element (48 x [500, 64] x
+  // [64, 500] 26.3 -> 16 us), K tails and C rows of any alignment among
+  // them; short chunks of whole tiles (1024^3 split four ways: 16 -> 17.5 us)
+  // keep the 32x32x16 kernel.
+  const bool k_tail = g.k_chunk % 64 != 0 || g.k % 64 != 0;
+  const bool only_mi16 = k_tail || !dma_pairs_ok(g);
+  if (g.k_chunk >= 16 * 64 || RAGGED || only_mi16) {
+    if (launch_mi16(g, LB, Mi16Tile{128, 128, mi16_stages128(g, grid), RAGGED}, grid, s)) return;
+    if (only_mi16) {
+      launch_gemm_bf16(g, 128, L_KCONTIG, LB, true, grid, s);
+      return;
+    }
   }
   switch (g.act) {
     case HMX_EPI_RELU: launch(gemm_bf16_dma64_kernel<LB, ACT_RELU, BF16, 4, 128, RAGGED, 128>, grid, 256, s, g); break;
@@ -1210,7 +915,7 @@ void launch_bf16_dma128_c(const GemmArgs& g, dim3 grid, hipStream_t s) {
 
 template <int LB>
 void launch_bf16_dma128_b(const GemmArgs& g, dim3 grid, hipStream_t s) {
-  const bool ragged = g.m % 128 != 0 || g.n % 128 != 0;
+  const bool ragged = g.m % 128 != 0 || g.n % 128 != 0 || g.k_chunk % 64 != 0 || g.k % 64 != 0;
   const bool bf16 = g.c_dtype == HMX_DTYPE_BF16;
   if (ragged) {
     if (bf16) launch_bf16_dma128_c<LB, true, true>(g, grid, s);
@@ -1255,7 +960,7 @@ void launch_gemm_bf16_dma_ta(const GemmArgs& g, int lb, dim3 grid, hipStream_t s
 }
 
 void launch_gemm_bf16_dma(const GemmArgs& g, int lb, dim3 grid, hipStream_t s) {
-  if (g.m % 256 != 0 || g.n % 256 != 0) {
+  if (g.m % 256 != 0 || g.n % 256 != 0 || g.k_chunk % 64 != 0 || g.k % 64 != 0) {
     const bool bf16 = g.c_dtype == HMX_DTYPE_BF16;
     if (lb == L_RCONTIG) {
       if (bf16) launch_bf16_dma_ragged<L_RCONTIG, true>(g, grid, s);
@@ -1270,25 +975,19 @@ void launch_gemm_bf16_dma(const GemmArgs& g, int lb, dim3 grid, hipStream_t s) {
     // The blocked VNNI layout [N/32, Kp/32, 16, 32, 2] is VNNI panels of 32.
     GemmArgs v = g;
     if (lb == L_BLOCKED_VNNI) v.b.panel = 32;
-    launch_bf16_dma_b<L_VNNI_PANELS, true>(v, grid, s);
+    launch_bf16_dma_b<L_VNNI_PANELS>(v, grid, s);
     return;
   }
   if (lb == L_PANELS) {
-    launch_bf16_dma_b<L_PANELS, true>(g, grid, s);
+    launch_bf16_dma_b<L_PANELS>(g, grid, s);
     return;
   }
   if (lb == L_BLOCKED) {
-    launch_bf16_dma_b<L_BLOCKED, true>(g, grid, s);
+    launch_bf16_dma_b<L_BLOCKED>(g, grid, s);
     return;
   }
-  const bool k64 = g.k_chunk % 64 == 0 && g.k % 64 == 0 && dma64_enabled();
-  if (lb == L_RCONTIG) {
-    if (k64) launch_bf16_dma_b<L_RCONTIG, true>(g, grid, s);
-    else launch_bf16_dma_b<L_RCONTIG, false>(g, grid, s);
-  } else {
-    if (k64) launch_bf16_dma_b<L_KCONTIG, true>(g, grid, s);
-    else launch_bf16_dma_b<L_KCONTIG, false>(g, grid, s);
-  }
+  if (lb == L_RCONTIG) launch_bf16_dma_b<L_RCONTIG>(g, grid, s);
+  else launch_bf16_dma_b<L_KCONTIG>(g, grid, s);
 }
 
 template <int NW, int D, int RB>

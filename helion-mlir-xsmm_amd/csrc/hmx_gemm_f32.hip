@@ -50,8 +50,8 @@ struct F32Loader {
         row = r0 + (item % (BR / 4)) * 4;
       }
       const bool fits = KC ? (row < o.rows && k + 4 <= k_end) : (row + 4 <= o.rows && k < k_end);
-      if (!GUARD || (o.vec && fits)) {
-        r[i] = *(const uint4*)(p + offset_of<L>(o, row, k));
+      if (!GUARD || fits) {
+        r[i] = load16(p + offset_of<L>(o, row, k));
       } else {
         float v[4];
 #pragma unroll

@@ -52,7 +52,6 @@ __device__ __forceinline__ void wait_vmem() {
   asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
 }
 
-__device__ __forceinline__ int swz_k(int r) { return ((r >> 1) & 3) ^ ((r >> 3) & 1); }
 __device__ __forceinline__ int swz_n(int r) { return ((r & 3) << 1) ^ ((r & 3) << 2); }
 __device__ __forceinline__ int swz64(int r) { return (r >> 1) & 7; }
 // Row-major B tiles of the 16x16x32 kernel: swz_n, with bit 3 of the K row

@@ -90,8 +90,11 @@ __device__ __forceinline__ void gemm_bf16_mi16_body(const GemmArgs& g, uint8_t* 
   const int split = blockIdx.y, batch = blockIdx.z;
   const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
   const int64_t k_begin = (int64_t)split * g.k_chunk;
-  const int64_t k_end = min(g.k, k_begin + g.k_chunk);
-  const int ktiles = (int)((k_end - k_begin) / BK);
+  // RAGGED also takes K chunks that are not whole stages: see zero_tail below.
+  // (k_chunk is K itself or whole stages: rounded up to even it still ends there.)
+  auto even = [](int64_t k) { return RAGGED ? (k + 1) & ~(int64_t)1 : k; };
+  const int64_t k_end = min(even(g.k), k_begin + even(g.k_chunk));
+  const int ktiles = (int)((k_end - k_begin + (RAGGED ? BK - 1 : 0)) / BK);
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -111,7 +114,7 @@ __device__ __forceinline__ void gemm_bf16_mi16_body(const GemmArgs& g, uint8_t* 
   // load's scalar offset is not range-checked, so each lane's whole row of A
   // (of K-contiguous B) sits in its vector offset, clamped to the last row,
   // row-major B's columns clamped to the last 8-column chunk, and the scalar
-  // offset holds only the K position. The duplicated rows and columns reach
+  // offset holds only the K position (row-major B: nothing). The duplicated rows and columns reach
   // only outputs that are never stored.
   auto kc_voff_clamped = [&](int64_t ld, int64_t row, int64_t rows, int par) {
     return (int32_t)((min(row, rows - 1) * ld + (slot ^ ((rr >> 1) | (par << 2))) * 8) * 2);
@@ -206,10 +209,45 @@ __device__ __forceinline__ void gemm_bf16_mi16_body(const GemmArgs& g, uint8_t* 
     soff_b = (int32_t)((n0 + wave * (BN / NW)) * g.b.ld * 2);
     blk_b = (int32_t)(8 * g.b.ld * 2);
   }
+  // A chunk that is not whole stages (RAGGED, K >= 64): its last stage holds
+  // the chunk's last 64 K values, so every load stays inside the operands'
+  // rows, and the 64 - `tail` of them that the stage before it held too are
+  // overwritten with zeros in LDS (zero_tail) once the stage has landed and a
+  // barrier published it; the caller adds the barrier that publishes that. An
+  // odd K counts one more: K-contiguous rows hold a zero there, and row-major
+  // B's row past the end is out of the buffer's range, which writes zeros to
+  // LDS. Every other stage runs the code of whole chunks: 4000^3 takes 98 us
+  // (the register-staged kernel, 261).
+  const int tail = (int)(k_end - k_begin) - (ktiles - 1) * BK;
+  auto zero_tail = [&](int stage) {
+    if constexpr (RAGGED) {
+      // The thread's index computed anew, so that nothing derived from it
+      // stays in registers through the loop for this.
+      int t = (int)threadIdx.x;
+      asm volatile("" : "+v"(t));
+      const int drop = BK - tail;
+      // One K-contiguous tile row per thread: its first drop / 8 pieces, and
+      // the first elements of the next.
+      auto zero = [&](uint8_t* tile, int r) {
+        for (int c = 0; c < (drop >> 3); ++c)
+          *(uint4*)(tile + r * ROWB + ((c ^ swz64(r)) << 4)) = make_uint4(0u, 0u, 0u, 0u);
+        uint16_t* piece = (uint16_t*)(tile + r * ROWB + (((drop >> 3) ^ swz64(r)) << 4));
+        for (int e = 0; e < (drop & 7); ++e) piece[e] = 0;
+      };
+      if (t < BM) zero(lds + stage * STAGE, t);
+      if constexpr (!BT) {
+        if (t < BN) zero(lds + stage * STAGE + A_BYTES, t);
+      } else {
+        for (int i = t * 16; i < drop * NROWB; i += NW * 64 * 16)
+          *(uint4*)(lds + stage * STAGE + A_BYTES + i) = make_uint4(0u, 0u, 0u, 0u);
+      }
+    }
+  };
   const uint32_t lds_w = __builtin_amdgcn_readfirstlane(lds_addr(lds)) + wave * LA * 1024;
   const uint32_t lds_wb = __builtin_amdgcn_readfirstlane(lds_addr(lds)) + A_BYTES + wave * LBN * 1024;
   auto dma = [&](int t, int q) {
-    const int64_t k0 = k_begin + (int64_t)min(t, ktiles - 1) * BK;
+    const int64_t k0 = RAGGED ? min(k_begin + (int64_t)t * BK, k_end - BK)
+                              : k_begin + (int64_t)min(t, ktiles - 1) * BK;
     const uint32_t st = lds_w + (uint32_t)((t & (S - 1)) * STAGE);
     const uint32_t sb = lds_wb + (uint32_t)((t & (S - 1)) * STAGE);
     if (q < LA) {
@@ -231,10 +269,14 @@ __device__ __forceinline__ void gemm_bf16_mi16_body(const GemmArgs& g, uint8_t* 
     } else {
       const int qb = q - LA;
       const int32_t kb = BT ? (int32_t)(k0 * g.b.ld * 2) : (int32_t)(k0 * 2);
-      // 256-byte B rows: load qb covers rows 4 qb .. 4 qb + 3 of the wave's,
-      // bit 3 of which is that of qb >> 1.
+      // 256-byte B rows: bit 3 of load qb's rows is that of qb >> 1.
       const bool hi = BT && BN == 128 ? (qb >> 1) & 1 : qb & 1;
-      lds_dma16(srd_b, hi ? voff_b1 : voff_b0, soff_b + qb * blk_b + kb, sb + qb * 1024);
+      const int32_t soff = (int32_t)((uint32_t)soff_b + (uint32_t)(qb * blk_b) + (uint32_t)kb);
+      // RAGGED: the K row is part of the range-checked offset (soff is uniform).
+      if constexpr (RAGGED)
+        lds_dma16(srd_b, (int32_t)((uint32_t)(hi ? voff_b1 : voff_b0) + (uint32_t)soff), 0, sb + qb * 1024);
+      else
+        lds_dma16(srd_b, hi ? voff_b1 : voff_b0, soff, sb + qb * 1024);
     }
   };
 
@@ -286,6 +328,10 @@ __device__ __forceinline__ void gemm_bf16_mi16_body(const GemmArgs& g, uint8_t* 
     for (int q = 0; q < LOADS; ++q) dma(u, q);
   wait_vmem<LOADS * (S - 1)>();  // stage 0 landed
   __syncthreads();
+  if (RAGGED && ktiles == 1 && tail < BK) {
+    zero_tail(0);
+    __syncthreads();
+  }
 #pragma unroll
   for (int i = 0; i < FM; ++i) fa[0][i] = a_read(0, 0, i);
 #pragma unroll
@@ -296,15 +342,22 @@ __device__ __forceinline__ void gemm_bf16_mi16_body(const GemmArgs& g, uint8_t* 
   // vmcnt 0), in a copy of the stage without them rather than behind a branch
   // per load; with four the barrier counts on S - 2 stages of loads behind
   // the next, which clamped reloads of the last stage keep.
-  auto stage = [&](int t, auto loads_c) {
-    constexpr bool LOADS_C = decltype(loads_c)::value;
+  // END_C: one of the last two stages (zero_tail's place); a copy of the stage
+  // too, since the branch alone cost the four-stage loop 20-50 %.
+  auto stage = [&](int t, auto loads_c, auto end_c) {
+    constexpr bool LOADS_C = decltype(loads_c)::value, END_C = decltype(end_c)::value;
     const int cur = t & (S - 1), nxt = (t + 1) & (S - 1);
 #pragma unroll
     for (int x = 0; x < SLOTS; ++x) {
       __builtin_amdgcn_sched_barrier(0);
       const int ks = x / NS, sub = x % NS;
-      if (x == BAR)
+      if (x == BAR) {
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(LOADS * (S - 2)) : "memory");
+        if (RAGGED && END_C && t == ktiles - 2 && tail < BK) {
+          zero_tail(nxt);
+          asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        }
+      }
       if (ks == 0 && sub < NF) {
         if (sub < FM) fa[1][sub] = a_read(cur, 1, sub);
         else fb[1][sub - FM] = b_read(cur, 1, sub - FM);
@@ -328,10 +381,14 @@ __device__ __forceinline__ void gemm_bf16_mi16_body(const GemmArgs& g, uint8_t* 
   };
   if constexpr (S == 2) {
     int t = 0;
-    for (; t < ktiles - S; ++t) stage(t, std::true_type{});
-    for (; t < ktiles; ++t) stage(t, std::false_type{});
+    for (; t < ktiles - S; ++t) stage(t, std::true_type{}, std::false_type{});
+    for (; t < ktiles; ++t) stage(t, std::false_type{}, std::true_type{});
+  } else if constexpr (RAGGED) {
+    int t = 0;
+    for (; t < ktiles - 2; ++t) stage(t, std::true_type{}, std::false_type{});
+    for (; t < ktiles; ++t) stage(t, std::true_type{}, std::true_type{});
   } else {
-    for (int t = 0; t < ktiles; ++t) stage(t, std::true_type{});
+    for (int t = 0; t < ktiles; ++t) stage(t, std::true_type{}, std::false_type{});
   }
   wait_vmem<0>();  // no load into LDS outlives the loop
 
@@ -480,11 +537,8 @@ __device__ __forceinline__ void gemm_bf16_mi16_body(const GemmArgs& g, uint8_t* 
     }
   } else {
     // f32 C straight from the fragments: a lane's four columns of a row are
-    // one 16-byte store where C's rows allow it (16-byte aligned, whole), else
-    // four 4-byte stores.
+    // one 16-byte store where they are whole, else four 4-byte stores.
     float* c = (float*)g.c + off;
-    const bool vec = ((((uintptr_t)g.c) & 15) == 0) && g.ldc % 4 == 0 && g.stride_c % 4 == 0 &&
-                     g.stride_split % 4 == 0;
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
       const int64_t col = n0 + col4_of(j);
@@ -497,12 +551,12 @@ __device__ __forceinline__ void gemm_bf16_mi16_body(const GemmArgs& g, uint8_t* 
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = activate<ACT>((acc[i][j][e] + cb[e]) * cs[e] + ch[e]);
         float* cp = c + row * g.ldc + col;
-        if ((!RAGGED || (row < g.m && col + 4 <= g.n)) && vec) {
+        if (!RAGGED || (row < g.m && col + 4 <= g.n)) {
           store_c(cp, Elem<float>::pack(v));
-        } else if (!RAGGED || row < g.m) {
+        } else if (row < g.m) {
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            if (!RAGGED || col + e < g.n) store_c32(cp + e, __float_as_uint(v[e]));
+            if (col + e < g.n) store_c32(cp + e, __float_as_uint(v[e]));
         }
       }
     }

@@ -61,9 +61,21 @@ constexpr DeviceShape kMi355x = {256, 8};
 DeviceShape current_device_shape();
 
 // Enqueues dst[c, r] = src[r, c] for 16-bit elements, src [rows, cols] with
-// row stride ld, dst [cols, rows] contiguous (hmx_pack.hip).
-void launch_transpose16(const void* src, void* dst, int64_t rows, int64_t cols, int64_t ld,
+// row stride ld, dst [cols, rows] with row stride dst_ld >= rows, zeros from
+// column `rows` on (hmx_pack.hip).
+void launch_transpose16(const void* src, void* dst, int64_t rows, int64_t cols, int64_t ld, int64_t dst_ld,
                         hipStream_t stream);
+
+// dst [batch, rows, dst_ld] = src [batch, rows, cols] (batch and row strides
+// `stride`, ld) of 16-bit elements, zeros from column `cols` on; dst 16-byte
+// aligned, dst_ld a multiple of 8.
+struct PadRows16 {
+  const void* src;
+  void* dst;
+  int64_t batch, stride, rows, cols, ld, dst_ld;
+};
+// Enqueues both copies in one launch (a batch of 0: none; hmx_pack.hip).
+void launch_pad_rows16(const PadRows16& a, const PadRows16& b, hipStream_t stream);
 
 inline bool valid_dtype(int dtype) {
   return dtype == HMX_DTYPE_F32 || dtype == HMX_DTYPE_BF16;

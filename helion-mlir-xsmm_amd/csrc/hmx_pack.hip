@@ -295,10 +295,11 @@ __global__ __launch_bounds__(256) void pack_vnni_t_kernel(const uint16_t* __rest
 }
 
 // Transpose of 16-bit elements, [rows, cols] (row stride ld) -> [cols, rows]
-// contiguous. Each lane moves an 8 x 8 block: eight 16-byte row loads, a
-// register transpose (v_perm_b32), eight 16-byte stores; a wave covers a
-// 64 x 64 tile with 128-byte segments on both sides. Edge blocks go element
-// by element.
+// (row stride dst_ld, zeros past `rows`). Each lane moves an 8 x 8 block: eight
+// 16-byte row loads at any alignment, a register transpose (v_perm_b32), eight
+// 16-byte stores; a wave covers a 64 x 64 tile with 128-byte segments on both
+// sides. Rows past the source's are zeros; only blocks that cross its last
+// columns, or the end of an unpadded destination row, go element by element.
 __device__ __forceinline__ uint32_t lo_pair(uint32_t x, uint32_t y) {
   return __builtin_amdgcn_perm(y, x, 0x05040100u);
 }
@@ -311,34 +312,79 @@ __device__ __forceinline__ uint32_t word(const uint4& v, int i) {
 
 __global__ __launch_bounds__(256) void transpose16_kernel(const uint16_t* __restrict__ src,
                                                           uint16_t* __restrict__ dst, int64_t rows,
-                                                          int64_t cols, int64_t ld, bool vec) {
+                                                          int64_t cols, int64_t ld, int64_t dst_ld) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t r0 = (int64_t)blockIdx.y * 64 + (lane & 7) * 8;
   const int64_t c0 = ((int64_t)blockIdx.x * 4 + wave) * 64 + (lane >> 3) * 8;
-  if (r0 >= rows || c0 >= cols) return;
+  if (r0 >= dst_ld || c0 >= cols) return;
   uint4 in[8];
-  const bool whole = vec && r0 + 8 <= rows && c0 + 8 <= cols;
-  if (whole) {
 #pragma unroll
-    for (int k = 0; k < 8; ++k) in[k] = *(const uint4*)(src + (r0 + k) * ld + c0);
-    // Output row j (source column c0 + j) holds source rows r0..r0+7.
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      uint4 o;
-      const int d = j >> 1;
-      if (j & 1) {
-        o = make_uint4(hi_pair(word(in[0], d), word(in[1], d)), hi_pair(word(in[2], d), word(in[3], d)),
-                       hi_pair(word(in[4], d), word(in[5], d)), hi_pair(word(in[6], d), word(in[7], d)));
+  for (int k = 0; k < 8; ++k) {
+    in[k] = make_uint4(0u, 0u, 0u, 0u);
+    if (r0 + k < rows) {
+      const uint16_t* p = src + (r0 + k) * ld + c0;
+      if (c0 + 8 <= cols) {
+        in[k] = load16(p);
       } else {
-        o = make_uint4(lo_pair(word(in[0], d), word(in[1], d)), lo_pair(word(in[2], d), word(in[3], d)),
-                       lo_pair(word(in[4], d), word(in[5], d)), lo_pair(word(in[6], d), word(in[7], d)));
+        uint32_t h[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) h[e] = c0 + e < cols ? p[e] : 0u;
+        in[k] = make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16));
       }
-      *(uint4*)(dst + (c0 + j) * rows + r0) = o;
     }
-  } else {
-    for (int j = 0; j < 8 && c0 + j < cols; ++j)
-      for (int k = 0; k < 8 && r0 + k < rows; ++k) dst[(c0 + j) * rows + r0 + k] = src[(r0 + k) * ld + c0 + j];
   }
+  // Output row j (source column c0 + j) holds source rows r0..r0+7.
+  const bool whole = r0 + 8 <= dst_ld;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    if (c0 + j >= cols) break;
+    uint4 o;
+    const int d = j >> 1;
+    if (j & 1) {
+      o = make_uint4(hi_pair(word(in[0], d), word(in[1], d)), hi_pair(word(in[2], d), word(in[3], d)),
+                     hi_pair(word(in[4], d), word(in[5], d)), hi_pair(word(in[6], d), word(in[7], d)));
+    } else {
+      o = make_uint4(lo_pair(word(in[0], d), word(in[1], d)), lo_pair(word(in[2], d), word(in[3], d)),
+                     lo_pair(word(in[4], d), word(in[5], d)), lo_pair(word(in[6], d), word(in[7], d)));
+    }
+    uint16_t* q = dst + (c0 + j) * dst_ld + r0;
+    if (whole) {
+      *reinterpret_cast<u32x4_any_t*>(q) = u32x4_any_t{o.x, o.y, o.z, o.w};
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (r0 + e < dst_ld) q[e] = (uint16_t)(word(o, e >> 1) >> (16 * (e & 1)));
+    }
+  }
+}
+
+// Rows copied into rows padded with zeros to a multiple of 8 elements
+// (PadRows16), for GEMM operands whose rows keep no 16-byte alignment: one
+// 16-byte load at any alignment and one aligned store per lane, bound by HBM.
+// Workgroups below `split` copy a, the others b.
+__global__ __launch_bounds__(256) void pad_rows16_kernel(PadRows16 a, PadRows16 b, unsigned split) {
+  const bool first = blockIdx.x < split;
+  const PadRows16& p = first ? a : b;
+  const int64_t per_row = p.dst_ld / 8;
+  const int64_t i = (int64_t)(first ? blockIdx.x : blockIdx.x - split) * 256 + threadIdx.x;
+  if (i >= p.batch * p.rows * per_row) return;
+  auto divide = [](int64_t n, int64_t d) {
+    return (uint64_t)n < 0xffffffffu ? (int64_t)((uint32_t)n / (uint32_t)d) : n / d;
+  };
+  const int64_t line = divide(i, per_row);
+  const int64_t col = (i - line * per_row) * 8;
+  const int64_t slice = p.batch == 1 ? 0 : divide(line, p.rows);
+  const uint16_t* src = (const uint16_t*)p.src + slice * p.stride + (line - slice * p.rows) * p.ld + col;
+  uint4 v;
+  if (col + 8 <= p.cols) {
+    v = load16(src);
+  } else {
+    uint32_t h[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) h[e] = col + e < p.cols ? src[e] : 0u;
+    v = make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16));
+  }
+  *reinterpret_cast<uint4*>((uint16_t*)p.dst + line * p.dst_ld + col) = v;
 }
 
 constexpr int64_t kMaxGridX = 0x7fffffff;
@@ -351,12 +397,15 @@ bool is_transposed(int kind) {
 
 }  // namespace
 
-void launch_transpose16(const void* src, void* dst, int64_t rows, int64_t cols, int64_t ld,
+void launch_transpose16(const void* src, void* dst, int64_t rows, int64_t cols, int64_t ld, int64_t dst_ld,
                         hipStream_t stream) {
-  const bool vec = aligned16(src) && aligned16(dst) && ld % 8 == 0 && rows % 8 == 0;
-  const dim3 grid((unsigned)ceil_div(cols, 256), (unsigned)ceil_div(rows, 64));
-  launch(transpose16_kernel, grid, 256, stream, (const uint16_t*)src, (uint16_t*)dst, rows, cols,
-         ld, vec);
+  const dim3 grid((unsigned)ceil_div(cols, 256), (unsigned)ceil_div(dst_ld, 64));
+  launch(transpose16_kernel, grid, 256, stream, (const uint16_t*)src, (uint16_t*)dst, rows, cols, ld, dst_ld);
+}
+
+void launch_pad_rows16(const PadRows16& a, const PadRows16& b, hipStream_t stream) {
+  auto blocks = [](const PadRows16& p) { return (unsigned)ceil_div(p.batch * p.rows * (p.dst_ld / 8), 256); };
+  launch(pad_rows16_kernel, dim3(blocks(a) + blocks(b)), 256, stream, a, b, blocks(a));
 }
 
 }  // namespace hmx
@@ -401,7 +450,7 @@ extern "C" int hmx_pack(int kind, int dtype, const void* src, int64_t rows, int6
   auto s = (hipStream_t)stream;
   if (kind == HMX_PACK_TRANSPOSE && dtype == HMX_DTYPE_BF16 && rows_pad == lrows &&
       cols_pad == lcols && rows > 0 && cols > 0) {
-    launch_transpose16(src, dst, rows, cols, ld, s);
+    launch_transpose16(src, dst, rows, cols, ld, rows, s);
     return check_launch("pack transpose");
   }
   if (kind == HMX_PACK_B_VNNI_PANELS_T && dtype == HMX_DTYPE_BF16 && panel % 64 == 0 && rows > 0 &&

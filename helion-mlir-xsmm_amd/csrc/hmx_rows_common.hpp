@@ -64,26 +64,10 @@ constexpr int kMaxBlock = kMaxWavesPerRow * kWave;
 constexpr int kProgBlock = 8 * kWave;
 
 // ---------------------------------------------------------------------------
-// 16 bytes at an address that keeps only its element type's alignment: rows of
-// any length are read and written as vectors (gfx950 takes 16-byte global
-// accesses at any element address; only the pieces that cross a cache line
-// cost a second request). Element-wise access of the same rows ran at a
-// quarter of the bandwidth: softmax of [24000, 501] bf16 32.6 -> 14.5 us,
-// RMSNorm of [16384, 3001] bf16 118 -> 42 us.
-typedef uint32_t u32x4_any_t __attribute__((ext_vector_type(4), aligned(2)));
-__device__ __forceinline__ uint4 load16(const void* p) {
-  const u32x4_any_t v = *reinterpret_cast<const u32x4_any_t*>(p);
-  return make_uint4(v[0], v[1], v[2], v[3]);
-}
-__device__ __forceinline__ uint4 load16_nt(const void* p) {
-  const u32x4_any_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any_t*>(p));
-  return make_uint4(v[0], v[1], v[2], v[3]);
-}
-__device__ __forceinline__ void store16_row(void* p, const uint4& v) {
-  __builtin_nontemporal_store(u32x4_any_t{v.x, v.y, v.z, v.w}, reinterpret_cast<u32x4_any_t*>(p));
-}
-
-// Row access. `tpr` threads share a row; thread `li` of them holds, as its
+// Row access: rows of any length and alignment in 16-byte vectors. Read
+// element by element where they kept no 16-byte alignment, the same rows ran
+// at a quarter of the bandwidth: softmax of [24000, 501] bf16 32.6 -> 14.5 us,
+// RMSNorm of [16384, 3001] bf16 118 -> 42 us. `tpr` threads share a row; thread `li` of them holds, as its
 // j-th vector, columns [(j * tpr + li) * EPV, ... + EPV): for each j the
 // threads read one contiguous tpr * EPV run, so every load instruction is
 // fully coalesced.
@@ -113,7 +97,7 @@ __device__ __forceinline__ void store_row(T* __restrict__ p, int n, int li, int 
   for (int j = 0; j < VPL; ++j) {
     const int64_t col = ((int64_t)j * tpr + li) * EPV;
     if (WHOLE || col + EPV <= n) {
-      store16_row(p + col, Elem<T>::pack(&v[j * EPV]));
+      store16_stream(p + col, Elem<T>::pack(&v[j * EPV]));
     } else {
 #pragma unroll
       for (int e = 0; e < EPV; ++e)
@@ -188,7 +172,7 @@ template <typename T, int EPV>
 __device__ __forceinline__ void store_chunk(T* __restrict__ p, int64_t n, int64_t col,
                                             const float (&v)[EPV]) {
   if (col + EPV <= n) {
-    store16_row(p + col, Elem<T>::pack(v));
+    store16_stream(p + col, Elem<T>::pack(v));
     return;
   }
 #pragma unroll

@@ -111,3 +111,39 @@ def test_ragged_loads_stay_inside_the_operands(m: int, n: int, k: int) -> None:
                     row = k0 + wave * 8 + 2 * qb + r
                     off = (row * n + col) * 2
                     assert off.min() >= 0 and (off + 16).max() <= span
+
+
+@pytest.mark.parametrize("k", [63, 64, 65, 66, 72, 100, 127, 128, 130, 191, 4004, 4100])
+@pytest.mark.parametrize("chunk", [64, 128, 1 << 20])
+def test_k_tail_stages_hold_each_k_once(k: int, chunk: int) -> None:
+    # K chunks that are not whole 64-element stages: the last stage of a chunk
+    # holds its last 64 K values, the ones the stage before it held are zeroed
+    # in LDS. K-contiguous rows (A; tagged with their K, row stride K rounded up
+    # to even, its last element 0 for odd K): every piece lies in its own row at
+    # 4-byte alignment, and the fragments' K values over all stages and chunks
+    # are 0 .. K - 1 once each. Row-major B: the rows fetched, of which row K
+    # (odd K) is the only one past the operand, at an offset past its range.
+    k2 = k + (k & 1)
+    row, slot = np.arange(16)[:, None], np.arange(8)[None, :]
+    swz = (row >> 1) & 7
+    seen = np.zeros((16, k2), dtype=int)
+    for begin in range(0, k2, chunk):
+        end = min(k2, begin + chunk)
+        stages = -(-(end - begin) // 64)
+        tail = (end - begin) - (stages - 1) * 64
+        for t in range(stages):
+            k0 = min(begin + t * 64, end - 64)
+            assert k0 >= 0 and k0 + 64 <= k2 and k0 % 2 == 0
+            assert all(r < k or (r == k and k % 2) for r in range(k0, k0 + 64))
+            lds = np.zeros((16, 8, 8), dtype=int)  # [row][slot][element]: K of the element
+            lds[row, slot] = (k0 + ((slot ^ swz) * 8))[..., None] + np.arange(8)
+            if t == stages - 1 and tail < 64:
+                drop = 64 - tail
+                for r in range(16):
+                    for c in range(drop >> 3):
+                        lds[r, c ^ ((r >> 1) & 7)] = -1
+                    lds[r, (drop >> 3) ^ ((r >> 1) & 7), : drop & 7] = -1
+            for r in range(16):
+                used = lds[r][lds[r] >= 0]
+                seen[r, used] += 1
+    assert (seen == 1).all()
