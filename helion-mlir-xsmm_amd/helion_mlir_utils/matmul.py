@@ -426,10 +426,17 @@ def bmm(a: Tensor, b: Tensor, *, out_dtype: torch.dtype | None = None, splits: i
         return c.zero_()
     if a.stride(2) != 1 or a.stride(1) < k:
         a = a.contiguous()
+    layout, ldb = native.B_ROW, b.stride(1)
     if b.stride(2) != 1 or b.stride(1) < n:
-        b = b.contiguous()
+        if b.stride(1) == 1 and b.stride(2) >= k:
+            # A transposed view, as attention scores pass their keys: read in
+            # place as the [N, K] matrices it views.
+            layout, ldb = native.B_TRANS, b.stride(2)
+        else:
+            b = b.contiguous()
+            ldb = b.stride(1)
     return _launch_gemm(
-        a, a.stride(1), False, b, b.stride(1), native.B_ROW, 0, 0, c, m, n, k,
+        a, a.stride(1), False, b, ldb, layout, 0, 0, c, m, n, k,
         batch=batch, stride_a=a.stride(0), stride_b=b.stride(0), stride_c=m * n,
         splits=0 if splits is None else int(splits),
     )
