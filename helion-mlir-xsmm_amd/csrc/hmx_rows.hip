@@ -78,8 +78,7 @@ __global__ __launch_bounds__(kMaxBlock) void softmax_stream(const T* x, T* y, in
   float mx = -INFINITY, base = 0.f, sum = 0.f;
   for (int64_t c = 0; c < chunks; ++c) {
     float top = mx;
-#pragma unroll
-    for (int u = 0; u < U; ++u) load_chunk<T, EPV>(xr, n, c * big + u * step + col0, v[u], -INFINITY);
+    load_chunks<T, EPV, U>(xr, n, c * big + col0, step, v, -INFINITY);
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -97,8 +96,7 @@ __global__ __launch_bounds__(kMaxBlock) void softmax_stream(const T* x, T* y, in
   if (mx > -INFINITY) sum *= exp_sub(mx, row_mx);
   const float inv = 1.f / row_sum_all(sum, red_sum, kMaxBlock);
   for (int64_t c = chunks - 1; c >= 0; --c) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) load_chunk<T, EPV>(xr, n, c * big + u * step + col0, v[u], 0.f);
+    load_chunks<T, EPV, U>(xr, n, c * big + col0, step, v, 0.f);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
 #pragma unroll
@@ -277,7 +275,14 @@ __global__ __launch_bounds__(kMaxBlock) void group_norm_walk(const T* x, T* y, G
   for (; row < rows; row += (int64_t)gridDim.y * rpw) {
     const int64_t off = (row * a.groups + g) * n;
     float v[VPL * EPV];
-    load_row<T, EPV, VPL, WHOLE>(x + off, (int)n, li, tpr, v, 0.f);
+    if constexpr (WHOLE) {
+      load_row<T, EPV, VPL, true>(x + off, (int)n, li, tpr, v, 0.f);
+    } else {
+#pragma unroll
+      for (int j = 0; j < VPL; ++j)
+        load_guarded<T, EPV, std::is_same_v<T, float>>(x + off, n, col_of<EPV>(j, li, tpr, 0),
+                                                       *reinterpret_cast<float (*)[EPV]>(&v[j * EPV]), 0.f);
+    }
     float s = 0.f;
 #pragma unroll
     for (int i = 0; i < VPL * EPV; ++i) s += v[i];
@@ -363,37 +368,102 @@ struct RowEpilogue {
   hmx_program prog;
 };
 
+// The products (or values) of EPV columns from `col` on, added to acc.
 template <typename T, int EPV, int MODE>
-__global__ __launch_bounds__(kBlock) void row_reduce(const T* x,
-                                                     const void* __restrict__ vec,
-                                                     T* y, int64_t m,
-                                                     int64_t n, RowEpilogue epi) {
-  const int64_t row = unit_index();
-  if (row >= m) return;
-  const int lane = threadIdx.x & (kWave - 1);
-  const T* xr = x + row * n;
-  const int64_t step = (int64_t)kWave * EPV;
-  float v[EPV];
+__device__ __forceinline__ void reduce_add(const float (&v)[EPV], const void* vec, int64_t n, int64_t col,
+                                           float& acc) {
+  if constexpr (MODE == 0) {
+#pragma unroll
+    for (int e = 0; e < EPV; ++e) acc += v[e];
+  } else {
+    float u[EPV];
+    if constexpr (MODE == 1) load_vec_run<float, EPV>((const float*)vec, n, col, u);
+    else load_chunk<T, EPV>((const T*)vec, n, col, u, 0.f);
+#pragma unroll
+    for (int e = 0; e < EPV; ++e) acc += v[e] * u[e];
+  }
+}
+
+__device__ __forceinline__ float reduce_finish(const RowEpilogue& epi, float s) {
+  return epi.act == HMX_EPI_PROGRAM ? run_program(epi.prog, s, 0.f) : apply_activation(epi.act, s, epi.arg);
+}
+
+// Rows of at most 64 x VPL vectors: `tpr` lanes a row (a power of two up to
+// 64), every load of the row in flight at once, several rows per wave where
+// they are short ([65536, 64] bf16, eight lanes a row: 10.6 us with a wave per row,
+// 2.9 us).
+template <typename T, int EPV, int MODE, int VPL>
+__global__ __launch_bounds__(kBlock) void row_reduce_short(const T* x, const void* __restrict__ vec, T* y, int64_t m,
+                                                           int64_t n, int tpr, RowEpilogue epi) {
+  const RowPos p = row_pos(tpr);
+  if (p.row >= m) return;
+  float v[VPL * EPV];
+  load_row<T, EPV, VPL>(x + p.row * n, (int)n, p.li, tpr, v, 0.f);
   float s = 0.f;
-  for (int64_t col = (int64_t)lane * EPV; col < n; col += step) {
-    load_chunk<T, EPV>(xr, n, col, v, 0.f);
-    if constexpr (MODE == 0) {
 #pragma unroll
-      for (int e = 0; e < EPV; ++e) s += v[e];
-    } else if constexpr (MODE == 1) {
-      float u[EPV];
-      load_vec_run<float, EPV>((const float*)vec, n, col, u);
+  for (int j = 0; j < VPL; ++j) {
+    const int64_t col = col_of<EPV>(j, p.li, tpr, 0);
+    if (col < n) reduce_add<T, EPV, MODE>(*reinterpret_cast<float (*)[EPV]>(&v[j * EPV]), vec, n, col, s);
+  }
+  for (int off = tpr >> 1; off > 0; off >>= 1) s += __shfl_xor(s, off, kWave);
+  s = reduce_finish(epi, s);
+  if (p.li == 0) Elem<T>::store(y + p.row, s);
+}
+
+// Longer rows: `wpr` waves share a row (a power of two; row_waves picks it), each summing every
+// wpr-th run of 64 vectors with four loads in flight per lane; their sums
+// meet in LDS and are added in wave order.
+template <typename T, int EPV, int MODE>
+__global__ __launch_bounds__(kMaxBlock) void row_reduce(const T* x, const void* __restrict__ vec, T* y, int64_t m,
+                                                        int64_t n, int wpr, RowEpilogue epi) {
+  constexpr int U = 4;
+  __shared__ float part[kMaxWavesPerRow];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & (kWave - 1), w = wave & (wpr - 1);
+  const int64_t row = (int64_t)blockIdx.x * ((blockDim.x >> 6) / wpr) + wave / wpr;
+  float s = 0.f;
+  if (row < m) {
+    const T* xr = x + row * n;
+    const int64_t step = (int64_t)wpr * kWave * EPV;
+    int64_t col = (int64_t)(w * kWave + lane) * EPV;
+    float acc[U] = {};
+    for (; col + (U - 1) * step + EPV <= n; col += U * step) {
+      uint4 raw[U], vr[MODE == 2 ? U : 1];
+      if constexpr (MODE == 2) {
 #pragma unroll
-      for (int e = 0; e < EPV; ++e) s += v[e] * u[e];
-    } else {
-      float u[EPV];
-      load_chunk<T, EPV>((const T*)vec, n, col, u, 0.f);
+        for (int u = 0; u < U; ++u) vr[u] = load16((const T*)vec + col + u * step);
+      }
 #pragma unroll
-      for (int e = 0; e < EPV; ++e) s += v[e] * u[e];
+      for (int u = 0; u < U; ++u) raw[u] = load16(xr + col + u * step);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        float v[EPV];
+        Elem<T>::unpack(raw[u], v);
+        if constexpr (MODE == 2) {
+          float w[EPV];
+          Elem<T>::unpack(vr[u], w);
+#pragma unroll
+          for (int e = 0; e < EPV; ++e) acc[u] += v[e] * w[e];
+        } else {
+          reduce_add<T, EPV, MODE>(v, vec, n, col + u * step, acc[u]);
+        }
+      }
     }
+    for (; col < n; col += step) {
+      float v[EPV];
+      load_chunk<T, EPV>(xr, n, col, v, 0.f);
+      reduce_add<T, EPV, MODE>(v, vec, n, col, acc[0]);
+    }
+    s = (acc[0] + acc[1]) + (acc[2] + acc[3]);
   }
   s = wave_sum(s);
-  s = epi.act == HMX_EPI_PROGRAM ? run_program(epi.prog, s, 0.f) : apply_activation(epi.act, s, epi.arg);
+  if (wpr > 1) {
+    if (lane == 0) part[wave] = s;
+    __syncthreads();
+    if (w != 0) return;
+    for (int q = 1; q < wpr; ++q) s += part[wave + q];
+  }
+  if (row >= m) return;
+  s = reduce_finish(epi, s);
   if (lane == 0) Elem<T>::store(y + row, s);
 }
 
@@ -414,6 +484,9 @@ __global__ __launch_bounds__(256) void column_partial_kernel(const T* x, float* 
   __shared__ float sums[TR][CB];
   const int tc = threadIdx.x % TC, tr = threadIdx.x / TC;
   const int64_t col = (int64_t)blockIdx.x * CB + tc * EPV;
+  // The vector across the last column starts earlier instead, at the row's
+  // last EPV columns; what it repeats is not kept.
+  const int64_t at = n >= EPV ? min(col, n - EPV) : col;
   const int64_t r0 = (int64_t)blockIdx.y * rows_per_chunk;
   const int64_t r1 = min(m, r0 + rows_per_chunk);
   float acc[EPV];
@@ -424,7 +497,7 @@ __global__ __launch_bounds__(256) void column_partial_kernel(const T* x, float* 
     for (; r + (U - 1) * TR < r1; r += U * TR) {
       float v[U][EPV];
 #pragma unroll
-      for (int u = 0; u < U; ++u) load_chunk<T, EPV>(x + (r + u * TR) * n, n, col, v[u], 0.f);
+      for (int u = 0; u < U; ++u) load_guarded<T, EPV>(x + (r + u * TR) * n, n, at, v[u], 0.f);
 #pragma unroll
       for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -432,13 +505,15 @@ __global__ __launch_bounds__(256) void column_partial_kernel(const T* x, float* 
     }
     for (; r < r1; r += TR) {
       float v[EPV];
-      load_chunk<T, EPV>(x + r * n, n, col, v, 0.f);
+      load_guarded<T, EPV>(x + r * n, n, at, v, 0.f);
 #pragma unroll
       for (int e = 0; e < EPV; ++e) acc[e] += v[e];
     }
   }
+  const int back = (int)(col - at);
 #pragma unroll
-  for (int e = 0; e < EPV; ++e) sums[tr][tc * EPV + e] = acc[e];
+  for (int e = 0; e < EPV; ++e)
+    if (e >= back && col < n) sums[tr][tc * EPV + e - back] = acc[e];
   __syncthreads();
   for (int k = threadIdx.x; k < CB; k += 256) {
     const int64_t c = (int64_t)blockIdx.x * CB + k;
@@ -496,7 +571,7 @@ __global__ __launch_bounds__(256) void elementwise_kernel(const T* x,
   for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * EPV; i < numel;
        i += stride) {
     float v[EPV];
-    load_chunk<T, EPV>(x, numel, i, v, 0.f);
+    load_guarded<T, EPV>(x, numel, i, v, 0.f);
 #pragma unroll
     for (int e = 0; e < EPV; ++e) {
       if (op == HMX_ELT_RELU)
@@ -606,6 +681,17 @@ template <typename F>
 void with_type(int dtype, F&& f) {
   if (dtype == HMX_DTYPE_BF16) f((uint16_t*)nullptr, IntC<8>{});
   else f((float*)nullptr, IntC<4>{});
+}
+
+// Waves per row of a row reduction: doubled while the rows' waves fill less
+// than half of what the CUs hold (16 of 32 waves each) and every lane keeps four
+// vectors of the row ([64, 32000] f32 43 -> 4.4 us, [16, 1000000] bf16 679 -> 21;
+// 8 or 32 waves as the goal measured the same).
+int row_waves(int64_t m, int64_t n, int epv) {
+  const int64_t enough = (int64_t)16 * current_device_shape().cus;
+  int wpr = 1;
+  while (wpr < kMaxWavesPerRow && m * wpr < enough && n >= (int64_t)wpr * 2 * kWave * epv * 4) wpr *= 2;
+  return wpr;
 }
 
 dim3 unit_grid(int64_t units) { return dim3((unsigned)ceil_div(units, kRowsPerBlock)); }
@@ -844,12 +930,34 @@ static int row_reduce_launch(const char* name, int mode, int dtype, const void* 
   with_type(dtype, [&](auto tp, auto epv_c) {
     using T = std::remove_pointer_t<decltype(tp)>;
     constexpr int EPV = decltype(epv_c)::value;
-    if (mode == 0)
-      launch(row_reduce<T, EPV, 0>, unit_grid(m), kBlock, s, (const T*)x, vec, (T*)y, m, n, epi);
-    else if (mode == 1)
-      launch(row_reduce<T, EPV, 1>, unit_grid(m), kBlock, s, (const T*)x, vec, (T*)y, m, n, epi);
-    else
-      launch(row_reduce<T, EPV, 2>, unit_grid(m), kBlock, s, (const T*)x, vec, (T*)y, m, n, epi);
+    auto with_mode = [&](auto&& f) {
+      if (mode == 0) f(IntC<0>{});
+      else if (mode == 1) f(IntC<1>{});
+      else f(IntC<2>{});
+    };
+    const int64_t vecs = ceil_div(n, EPV);
+    if (vecs <= 4 * kWave) {
+      int tpr = 1;
+      while (tpr < kWave && tpr < vecs) tpr *= 2;
+      const dim3 grid((unsigned)ceil_div(m, kBlock / tpr));
+      with_mode([&](auto mode_c) {
+        constexpr int MODE = decltype(mode_c)::value;
+        auto go = [&](auto vpl_c) {
+          launch(row_reduce_short<T, EPV, MODE, decltype(vpl_c)::value>, grid, kBlock, s, (const T*)x, vec, (T*)y, m,
+                 n, tpr, epi);
+        };
+        if (vecs <= kWave) go(IntC<1>{});
+        else if (vecs <= 2 * kWave) go(IntC<2>{});
+        else go(IntC<4>{});
+      });
+      return;
+    }
+    const int wpr = row_waves(m, n, EPV);
+    const int block = std::max(kRowsPerBlock, wpr) * kWave;
+    const dim3 grid((unsigned)ceil_div(m, block / kWave / wpr));
+    with_mode([&](auto mode_c) {
+      launch(row_reduce<T, EPV, decltype(mode_c)::value>, grid, block, s, (const T*)x, vec, (T*)y, m, n, wpr, epi);
+    });
   });
   return check_launch(name);
 }
@@ -871,12 +979,17 @@ int hmx_matvec(int dtype, const void* a, const void* x, void* y, int64_t m, int6
   return row_reduce_launch("matvec", 2, dtype, a, x, y, m, k, HMX_EPI_IDENTITY, 0.f, nullptr, stream);
 }
 
-// Row chunks of a column sum: about 2048 workgroups, at least 256 rows each.
 // Row chunks of pass 1: about 1024 workgroups over the column blocks of
-// 512 columns, at least 256 rows per chunk.
+// 512 columns, at most 256 (the second pass adds a column's chunks in order: 1024
+// of them took [65536, 512] f32 from 26 to 32 us) of at least one batch of rows
+// per thread (eight; fewer threads across leave more down the rows), and one
+// chunk, with no second pass, for up to two batches. With at least 256 rows per
+// chunk, [4096, 4096] bf16 ran 128 workgroups: 26.8 -> 10 us.
 static void column_chunks(int64_t m, int64_t n, int64_t& chunks, int64_t& rows_per_chunk) {
   const int64_t blocks = std::max<int64_t>(1, ceil_div(n, 512));
-  chunks = std::max<int64_t>(1, std::min(ceil_div(1024, blocks), ceil_div(m, 256)));
+  const int64_t batch = n <= 64 ? 256 : n <= 128 ? 128 : n <= 256 ? 64 : 32;
+  chunks = std::max<int64_t>(1, std::min(std::min<int64_t>(ceil_div(1024, blocks), 256), ceil_div(m, batch)));
+  if (batch == 32 && m <= 2 * batch) chunks = 1;
   rows_per_chunk = ceil_div(m, chunks);
   chunks = rows_per_chunk > 0 ? ceil_div(m, rows_per_chunk) : 1;
 }

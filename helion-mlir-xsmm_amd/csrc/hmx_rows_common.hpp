@@ -64,29 +64,84 @@ constexpr int kMaxBlock = kMaxWavesPerRow * kWave;
 constexpr int kProgBlock = 8 * kWave;
 
 // ---------------------------------------------------------------------------
-// Row access: rows of any length and alignment in 16-byte vectors. Read
-// element by element where they kept no 16-byte alignment, the same rows ran
-// at a quarter of the bandwidth: softmax of [24000, 501] bf16 32.6 -> 14.5 us,
-// RMSNorm of [16384, 3001] bf16 118 -> 42 us. `tpr` threads share a row; thread `li` of them holds, as its
+// 16-byte vectors of a row of n elements, at any column and alignment, with no
+// branch around the load (loaded and unpacked behind one, each vector's load
+// is waited for before the next is issued: softmax of [24000, 501] bf16 14.5
+// -> 11.4 us, RMSNorm of [16384, 3001] 42 -> 36, [4000, 20000] softmax 55 -> 50). A vector that crosses the row's
+// end is read from the row's last EPV elements instead (raw_vec), and finish_vec
+// moves its elements to where they belong, `fill` past the end. Rows shorter
+// than a vector are gathered.
+template <typename T>
+__device__ __forceinline__ uint32_t elem_bits(float v) {
+  return sizeof(T) == 2 ? f32_to_bf16_bits(v) : __float_as_uint(v);
+}
+
+template <typename T, int EPV, bool NT = false>
+__device__ __forceinline__ uint4 raw_vec(const T* __restrict__ p, int64_t n, int64_t col, float fill) {
+  if (n >= EPV) {
+    const T* q = p + min(col, n - EPV);
+    return NT ? load16_nt(q) : load16(q);
+  }
+  float v[EPV];
+#pragma unroll
+  for (int e = 0; e < EPV; ++e) v[e] = col + e < n ? Elem<T>::load(p + col + e) : fill;
+  return Elem<T>::pack(v);
+}
+
+template <typename T, int EPV>
+__device__ __forceinline__ uint4 finish_vec(uint4 r, int64_t n, int64_t col, float fill) {
+  if (n < EPV || col + EPV <= n) return r;
+  const int back = (int)min(col + EPV - n, (int64_t)EPV);  // elements that belong to earlier vectors
+  const uint32_t f = elem_bits<T>(fill);
+  if constexpr (sizeof(T) == 2) {
+    const uint64_t ff = (uint64_t)(f | (f << 16)) * 0x100000001ull;
+    uint64_t lo = r.x | ((uint64_t)r.y << 32), hi = r.z | ((uint64_t)r.w << 32);
+    int k = back;
+    if (k >= 4) {
+      lo = hi;
+      hi = ff;
+      k -= 4;
+    }
+    if (k >= 4) {
+      lo = ff;
+      k = 0;
+    }
+    if (k > 0) {
+      lo = (lo >> (16 * k)) | (hi << (64 - 16 * k));
+      hi = (hi >> (16 * k)) | (ff << (64 - 16 * k));
+    }
+    return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+  } else {
+    const uint32_t x = back == 1 ? r.y : back == 2 ? r.z : back == 3 ? r.w : f;
+    const uint32_t y = back == 1 ? r.z : back == 2 ? r.w : f;
+    return make_uint4(x, y, back == 1 ? r.w : f, f);
+  }
+}
+
+// Row access. `tpr` threads share a row; thread `li` of them holds, as its
 // j-th vector, columns [(j * tpr + li) * EPV, ... + EPV): for each j the
 // threads read one contiguous tpr * EPV run, so every load instruction is
-// fully coalesced.
+// fully coalesced. Read element by element where they kept no 16-byte
+// alignment, rows ran at a quarter of the bandwidth: softmax of [24000, 501]
+// bf16 32.6 -> 11.4 us, RMSNorm of [16384, 3001] bf16 118 -> 36 us.
 // WHOLE: n == tpr * VPL * EPV, every vector is in the row (no guards).
 template <typename T, int EPV, int VPL, bool WHOLE = false>
 __device__ __forceinline__ void load_row(const T* __restrict__ p, int n, int li, int tpr,
                                          float (&v)[VPL * EPV], float fill) {
+  // f32 rows: non-temporal loads measure 2-3% more bandwidth on
+  // [32768, 4096] softmax/RMSNorm; for bf16 rows they cost 8-12%.
+  constexpr bool NT = std::is_same_v<T, float>;
+  uint4 raw[VPL];
 #pragma unroll
   for (int j = 0; j < VPL; ++j) {
     const int col = (j * tpr + li) * EPV;
-    if (WHOLE || col + EPV <= n) {
-      // f32 rows: non-temporal loads measure 2-3% more bandwidth on
-      // [32768, 4096] softmax/RMSNorm; for bf16 rows they cost 8-12%.
-      const uint4 raw = std::is_same_v<T, float> ? load16_nt(p + col) : load16(p + col);
-      Elem<T>::unpack(raw, &v[j * EPV]);
-    } else {
+    if constexpr (WHOLE) raw[j] = NT ? load16_nt(p + col) : load16(p + col);
+    else raw[j] = raw_vec<T, EPV, NT>(p, n, col, fill);
+  }
 #pragma unroll
-      for (int e = 0; e < EPV; ++e) v[j * EPV + e] = (col + e < n) ? Elem<T>::load(p + col + e) : fill;
-    }
+  for (int j = 0; j < VPL; ++j) {
+    if constexpr (!WHOLE) raw[j] = finish_vec<T, EPV>(raw[j], n, (j * tpr + li) * EPV, fill);
+    Elem<T>::unpack(raw[j], &v[j * EPV]);
   }
 }
 
@@ -160,8 +215,29 @@ __device__ __forceinline__ float row_max_all(float v, float* slot, int tpr) {
 template <typename T, int EPV>
 __device__ __forceinline__ void load_chunk(const T* __restrict__ p, int64_t n, int64_t col,
                                            float (&v)[EPV], float fill) {
+  Elem<T>::unpack(finish_vec<T, EPV>(raw_vec<T, EPV>(p, n, col, fill), n, col, fill), v);
+}
+// U of them, `step` columns apart, their loads in flight together.
+template <typename T, int EPV, int U>
+__device__ __forceinline__ void load_chunks(const T* __restrict__ p, int64_t n, int64_t col, int64_t step,
+                                            float (&v)[U][EPV], float fill) {
+  uint4 raw[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) raw[u] = raw_vec<T, EPV>(p, n, col + u * step, fill);
+#pragma unroll
+  for (int u = 0; u < U; ++u) Elem<T>::unpack(finish_vec<T, EPV>(raw[u], n, col + u * step, fill), v[u]);
+}
+
+// One vector behind a branch: as compiled, it has arrived before the next one is
+// asked for. Kernels that stream rows through few registers and many waves run
+// faster that way than with every load in flight: column_sum of [65536, 512]
+// f32 39.8 -> 26 us, [32768, 4096] bf16 51.5 -> 43.6; LayerNorm of [4096,
+// 11008] bf16 (walked) 54 -> 39.6.
+template <typename T, int EPV, bool NT = false>
+__device__ __forceinline__ void load_guarded(const T* __restrict__ p, int64_t n, int64_t col, float (&v)[EPV],
+                                             float fill) {
   if (col + EPV <= n) {
-    Elem<T>::unpack(load16(p + col), v);
+    Elem<T>::unpack(NT ? load16_nt(p + col) : load16(p + col), v);
     return;
   }
 #pragma unroll

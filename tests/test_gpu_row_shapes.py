@@ -94,3 +94,36 @@ def test_group_norm_group_sizes(gpu_device, m: int, groups: int, gs: int, dtype:
     assert_close(to_np(U.group_norm(x, groups, w, b, 1e-5)), ref, rtol, atol)
     added = R.group_norm(xs, groups, ws, bs, 1e-5, extra=es, extra_op="add", out=dtype)
     assert_close(to_np(U.group_norm(x, groups, w, b, 1e-5, torch.add, e)), added, rtol, atol)
+
+
+# Short rows (lanes of a wave share them), rows of one to four vectors a lane
+# (bf16: 512, 1024, 2048 columns), longer ones by 1 to 16 waves with the
+# unrolled loop's remainder, few rows and many.
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize(("m", "n"), [(3, 1), (300, 7), (1000, 65), (70, 511), (5, 1025), (9, 2047), (3, 2049),
+                                     (20000, 2100), (2, 16391), (1, 70001)])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_row_reductions_of_every_layout(gpu_device, m: int, n: int, dtype: str, offset: int) -> None:
+    x = _rows(m, n, dtype, gpu_device, offset)
+    v = _rows(1, n, "f32", gpu_device, offset)[0]
+    col = _rows(n, 1, dtype, gpu_device, offset)
+    xs = to_np(x).astype(np.float64)
+    # f32 sums of n terms of size |x| |v|: n eps in the worst order, of which a
+    # pairwise-like one shows sqrt(n); bf16 adds its rounding of the result.
+    scale = np.sqrt(n) * 4
+    rtol, atol = (1e-5, 2.0**-23 * np.sqrt(n) * scale) if dtype == "f32" else (2.0**-8, 2.0**-23 * n * 4)
+    for got, w in ((U.row_sum(x), np.ones(n)), (U.row_dot(x, v), to_np(v)), (U.matvec(x, col), to_np(col)[:, 0])):
+        assert_close(to_np(got), xs @ w.astype(np.float64)[:, None], rtol, atol)
+
+
+# One chunk, two, many, up to the limit on chunks; the vector across the last
+# column of every block width; one row.
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize(("m", "n"), [(1, 3), (64, 515), (65, 513), (200, 63), (1000, 129), (5000, 257), (40000, 517),
+                                     (33, 40001)])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_column_sum_chunks(gpu_device, m: int, n: int, dtype: str, offset: int) -> None:
+    x = _rows(m, n, dtype, gpu_device, offset)
+    got = U.column_sum(x)
+    assert torch.equal(got, U.column_sum(x))
+    assert_close(to_np(got), to_np(x).astype(np.float64).sum(0), 1e-5, 2.0**-23 * m * 4)
