@@ -57,8 +57,9 @@ constexpr TileChoice kF32Tiles[] = {{128, 128, 32}, {64, 64, 32}};
 // The f32 tile long-K split-K products of whole 256 x 256 tiles take (see
 // make_plan): one workgroup per CU reading each operand once.
 constexpr TileChoice kF32Big = {256, 256, 32};
-// The skinny kernel's plan (see skinny_shape).
+// The skinny and streaming kernels' plans (see skinny_shape, stream_shape).
 constexpr TileChoice kSkinny = {32, 32, 64};
+constexpr TileChoice kStream = {32, 64, 32};
 
 int layout_code(int b_layout) {
   switch (b_layout) {
@@ -95,6 +96,9 @@ struct Plan {
   // M <= 64 against B [N, K]: the skinny kernel (tile 32 x 32 x 64, no
   // split, no workspace).
   bool skinny;
+  // M <= 32 against a packed B: the streaming kernel (tile 32 x 64 x 32, no
+  // split, no workspace).
+  bool stream;
 };
 
 // f32 products whose tiles fill at most a quarter of the CUs are bound by
@@ -180,6 +184,17 @@ bool skinny_shape(int ab_dtype, int64_t m, int64_t k, int64_t batch, int trans_a
          !trans_a && b_layout == HMX_B_TRANS && splits <= 1 && (no_tile || skinny_tile);
 }
 
+// Products of at most 32 rows of row-major bf16 A (batch 1, K a multiple of
+// 32, from 256 on: 8 waves of one step) against a packed B take the streaming
+// kernel, unless the caller asks for K splits or names another tile.
+bool stream_shape(int ab_dtype, int64_t m, int64_t k, int64_t batch, int trans_a, int b_layout, int splits,
+                  int tile_m, int tile_n, int tile_k) {
+  const bool no_tile = tile_m <= 0 && tile_n <= 0 && tile_k <= 0;
+  const bool own_tile = tile_m == kStream.bm && tile_n == kStream.bn && tile_k == kStream.bk;
+  return ab_dtype == HMX_DTYPE_BF16 && m >= 1 && m <= kStream.bm && k >= 256 && k % 32 == 0 && batch == 1 &&
+         !trans_a && b_layout != HMX_B_ROW && b_layout != HMX_B_TRANS && splits <= 1 && (no_tile || own_tile);
+}
+
 bool dma_enabled();
 
 // Whether an unsplit bf16 launch of this shape takes a direct-to-LDS kernel,
@@ -215,8 +230,9 @@ int make_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int64_t batch, int 
       epilogue == HMX_EPI_IDENTITY || epilogue == HMX_EPI_RELU || epilogue == HMX_EPI_SILU;
   plan.skinny = !program &&
                 skinny_shape(ab_dtype, m, k, batch, trans_a, b_layout, splits, tile_m, tile_n, tile_k);
-  if (plan.skinny) {
-    plan.tile = kSkinny;
+  plan.stream = !program && stream_shape(ab_dtype, m, k, batch, trans_a, b_layout, splits, tile_m, tile_n, tile_k);
+  if (plan.skinny || plan.stream) {
+    plan.tile = plan.skinny ? kSkinny : kStream;
     plan.splits = 1;
     plan.k_chunk = k;
     plan.transpose_b = plan.transpose_a = plan.pad_a = plan.pad_b = false;
@@ -262,7 +278,6 @@ int make_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int64_t batch, int 
   const TileChoice* table = bf16 ? kBf16Tiles : kF32Tiles;
   const int count = bf16 ? (int)(sizeof(kBf16Tiles) / sizeof(TileChoice))
                          : (int)(sizeof(kF32Tiles) / sizeof(TileChoice));
-  // Packed B layouts are instantiated for the first tile only.
   const bool packed = b_layout != HMX_B_ROW && b_layout != HMX_B_TRANS;
   int pick = -1;
   // Whole 256 x 256 tiles of row-major A and an unpacked B: what the big f32
@@ -309,7 +324,9 @@ int make_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int64_t batch, int 
         big_tiles >= cus)
       pick = -2;
   }
-  if (packed && bf16) pick = 0;
+  // bf16 packed B on 128 x 128 tiles, where the direct-to-LDS kernel reads it
+  // (launches it cannot take go to the 256 x 256 register-staged kernel).
+  if (packed && bf16 && (k % 64 != 0 || n % 128 != 0 || program)) pick = 0;
   plan.tile = pick == -2 ? kF32Big : table[pick];
   const int64_t tiles = ceil_div(m, plan.tile.bm) * ceil_div(n, plan.tile.bn) * batch;
   const int64_t kt = ceil_div(k, plan.tile.bk);
@@ -395,7 +412,7 @@ bool dma_direct_ok(const GemmArgs& g) {
 }
 
 // The kernel families a launch can take.
-enum class Kernel { SKINNY, SKINNY_TILES, DMA, DMA_TA, DMA128, BF16, F32_DMA, F32 };
+enum class Kernel { SKINNY, SKINNY_TILES, STREAM, DMA, DMA_TA, DMA128, BF16, F32_DMA, F32 };
 
 // Whether a family runs epilogue programs fused (the direct-to-LDS bf16
 // kernels, through their LDS-staged epilogue); the others leave them to the
@@ -415,6 +432,7 @@ Kernel select_kernel(const GemmArgs& g, const Plan& plan, int ab_dtype, int la, 
   // The direct-to-LDS loads take 16-byte pieces at any 4-byte alignment.
   const bool words = (g.a.vec || g.a.word) && (g.b.vec || (plain_b && g.b.word)) && bytes_ok;
   if (plan.skinny) return aligned && dma_enabled() ? Kernel::SKINNY : Kernel::SKINNY_TILES;
+  if (plan.stream) return Kernel::STREAM;
   if (ab_dtype == HMX_DTYPE_BF16) {
     const TileChoice t = plan.tile;
     const bool k64 = g.k % 64 == 0 && plan.k_chunk % 64 == 0;
@@ -425,13 +443,17 @@ Kernel select_kernel(const GemmArgs& g, const Plan& plan, int ab_dtype, int la, 
     const bool k_ok = k64 || (mi16 && plain_b && la == L_KCONTIG && g.k >= 63 && g.act != HMX_EPI_PROGRAM);
     // Whole 256 x 256 tiles, or ragged M, N and K with B K-contiguous or
     // row-major.
-    const bool dma_shape = words && k_ok && (whole || plain_b);
+    // Packed B's padded columns fill whole tiles (M is ragged then); programs
+    // only on whole 256 x 256 ones.
+    const bool packed_b = !plain_b && gemm_bf16_dma_packed_ok(g, lb) &&
+                          (whole || (mi16 && g.b.rows % t.bn == 0 && g.act != HMX_EPI_PROGRAM));
+    const bool dma_shape = words && k_ok && (plain_b || packed_b);
     const bool ok = (dma_direct_ok(g) || (mi16 && g.k > 0)) && dma_enabled();
-    if (t.bm == 256 && dma_shape && la == L_KCONTIG && (plain_b || gemm_bf16_dma_packed_ok(g, lb)) && ok)
-      return Kernel::DMA;
+    if (t.bm == 256 && dma_shape && la == L_KCONTIG && ok) return Kernel::DMA;
     if (t.bm == 256 && la == L_RCONTIG && whole && aligned && plain_b && dma_direct_ok(g) && dma_enabled())
       return Kernel::DMA_TA;
-    if (t.bm == 128 && dma_shape && la == L_KCONTIG && plain_b && ok) return Kernel::DMA128;
+    if (t.bm == 128 && dma_shape && la == L_KCONTIG && ok && (plain_b || (mi16 && g.act != HMX_EPI_PROGRAM)))
+      return Kernel::DMA128;
     return Kernel::BF16;
   }
   const bool guard = !(whole && aligned);
@@ -725,7 +747,7 @@ int gemm_impl(int ab_dtype, int c_dtype, const void* a, int64_t lda, int trans_a
       const char* e = getenv("HMX_GEMM_STAGGER");
       return !(e && e[0] == '0');
     }();
-    g.k_stagger = stagger && plan.splits > 1 && tiles_m * tiles_n == 1 && k % 64 == 0;
+    g.k_stagger = stagger && plan.splits > 1 && tiles_m * tiles_n == 1 && k % 64 == 0 && !packed;
     g.c = partials;
     g.c_dtype = HMX_DTYPE_F32;
     g.ldc = n;
@@ -749,6 +771,11 @@ int gemm_impl(int ab_dtype, int c_dtype, const void* a, int64_t lda, int trans_a
       g.tiles_m = 1;
       g.tiles_n = (int)ceil_div(n, 128);
       launch_gemm_bf16(g, 128, la, lb_run, true, dim3((unsigned)g.tiles_n, 1, 1), s);
+      break;
+    case Kernel::STREAM:
+      // (Any alignment; 32-bit offsets.)
+      if (bytes_ok) launch_gemm_bf16_stream(g, lb_run, s);
+      else launch_gemm_bf16(g, 256, la, lb_run, true, grid, s);
       break;
     case Kernel::DMA: {
       const int64_t n1 = whole && (lb_run == L_KCONTIG || lb_run == L_RCONTIG) && plan.splits == 1 &&

@@ -439,6 +439,9 @@ bool gemm_mi16_ok(const GemmArgs& g);
 bool launch_mi16(const GemmArgs& g, int lb, Mi16Tile t, dim3 grid, hipStream_t s);
 bool launch_mi16_nt(const GemmArgs& g, Mi16Tile t, dim3 grid, hipStream_t s);
 bool launch_mi16_nn(const GemmArgs& g, Mi16Tile t, dim3 grid, hipStream_t s);
+bool launch_mi16_vnni(const GemmArgs& g, Mi16Tile t, dim3 grid, hipStream_t s);
+bool launch_mi16_panels(const GemmArgs& g, Mi16Tile t, dim3 grid, hipStream_t s);
+bool launch_mi16_blocked(const GemmArgs& g, Mi16Tile t, dim3 grid, hipStream_t s);
 bool launch_mi16_rounds(const GemmArgs& head, const GemmArgs& rest, int lb, unsigned head_blocks,
                         unsigned rest_blocks, hipStream_t s);
 bool launch_mi16_rounds_nt(const GemmArgs& head, const GemmArgs& rest, unsigned head_blocks, unsigned rest_blocks,
@@ -470,6 +473,9 @@ void launch_gemm_bf16_dma128(const GemmArgs& g, int lb, dim3 grid, hipStream_t s
 // 64, operand spans below 2^31 bytes, 16-byte aligned rows; one workgroup per
 // 32 columns of C, K split over its waves, any epilogue, C bf16 or f32.
 void launch_gemm_bf16_skinny(const GemmArgs& g, hipStream_t s);
+// hmx_gemm_stream.hip: M <= 32, row-major A, packed B, batch 1, K a multiple of 32, operand spans below 2^31 bytes; any epilogue but programs,
+// C bf16 or f32.
+void launch_gemm_bf16_stream(const GemmArgs& g, int lb, hipStream_t s);
 // Whether the 64-wide direct-to-LDS kernel reads this packed B in place
 // (VNNI panels, blocked VNNI, K-major panels, 32 x 32 blocks).
 bool gemm_bf16_dma_packed_ok(const GemmArgs& g, int lb);

@@ -783,6 +783,35 @@ void launch_bf16_dma_b(const GemmArgs& g, dim3 grid, hipStream_t s) {
 
 }  // namespace
 
+// The 16x16x32 MFMA kernel unless the environment sets HMX_GEMM_MFMA=32 (the
+// 32x32x16 kernel, for comparison); it does not stagger K walks.
+bool gemm_mi16_ok(const GemmArgs& g) {
+  static const bool on = [] {
+    const char* e = getenv("HMX_GEMM_MFMA");
+    return !(e && e[0] == '3');
+  }();
+  return on && !g.k_stagger;
+}
+
+bool launch_mi16(const GemmArgs& g, int lb, Mi16Tile t, dim3 grid, hipStream_t s) {
+  if (!gemm_mi16_ok(g)) return false;
+  switch (lb) {
+    case L_KCONTIG: return launch_mi16_nt(g, t, grid, s);
+    case L_RCONTIG: return launch_mi16_nn(g, t, grid, s);
+    case L_VNNI_PANELS: return launch_mi16_vnni(g, t, grid, s);
+    case L_PANELS: return launch_mi16_panels(g, t, grid, s);
+    case L_BLOCKED: return launch_mi16_blocked(g, t, grid, s);
+  }
+  return false;
+}
+
+bool launch_mi16_rounds(const GemmArgs& head, const GemmArgs& rest, int lb, unsigned head_blocks,
+                        unsigned rest_blocks, hipStream_t s) {
+  if (!gemm_mi16_ok(head) || !gemm_mi16_ok(rest)) return false;
+  return lb == L_KCONTIG ? launch_mi16_rounds_nt(head, rest, head_blocks, rest_blocks, s)
+                         : launch_mi16_rounds_nn(head, rest, head_blocks, rest_blocks, s);
+}
+
 bool dma_pairs_ok(const GemmArgs& g) {
   return g.c_dtype != HMX_DTYPE_BF16 ||
          (g.ldc % 2 == 0 && g.stride_c % 2 == 0 && g.stride_split % 2 == 0 && (((uintptr_t)g.c) & 3) == 0);
@@ -926,7 +955,25 @@ void launch_bf16_dma128_b(const GemmArgs& g, dim3 grid, hipStream_t s) {
   }
 }
 
+// A ragged product of packed B on tiles of bm x bm, or, where its epilogue could
+// not be compiled at run time, on the register-staged kernel.
+void launch_packed_ragged(const GemmArgs& g, int lb, int bm, dim3 grid, hipStream_t s) {
+  GemmArgs v = g;
+  int l = lb;
+  if (lb == L_BLOCKED_VNNI) {
+    // [N/32, Kp/32, 16, 32, 2] is VNNI panels of 32.
+    v.b.panel = 32;
+    l = L_VNNI_PANELS;
+  }
+  if (launch_mi16(v, l, Mi16Tile{bm, bm, bm == 128 ? mi16_stages128(g, grid) : 2, true}, grid, s)) return;
+  launch_gemm_bf16(g, 256, L_KCONTIG, lb, true, grid, s);
+}
+
 void launch_gemm_bf16_dma128(const GemmArgs& g, int lb, dim3 grid, hipStream_t s) {
+  if (lb != L_RCONTIG && lb != L_KCONTIG) {
+    launch_packed_ragged(g, lb, 128, grid, s);
+    return;
+  }
   if (lb == L_RCONTIG)
     launch_bf16_dma128_b<L_RCONTIG>(g, grid, s);
   else
@@ -960,6 +1007,10 @@ void launch_gemm_bf16_dma_ta(const GemmArgs& g, int lb, dim3 grid, hipStream_t s
 }
 
 void launch_gemm_bf16_dma(const GemmArgs& g, int lb, dim3 grid, hipStream_t s) {
+  if (lb != L_RCONTIG && lb != L_KCONTIG && (g.m % 256 != 0 || g.n % 256 != 0)) {
+    launch_packed_ragged(g, lb, 256, grid, s);
+    return;
+  }
   if (g.m % 256 != 0 || g.n % 256 != 0 || g.k_chunk % 64 != 0 || g.k % 64 != 0) {
     const bool bf16 = g.c_dtype == HMX_DTYPE_BF16;
     if (lb == L_RCONTIG) {

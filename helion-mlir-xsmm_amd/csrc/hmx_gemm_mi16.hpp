@@ -57,13 +57,13 @@ __device__ __forceinline__ void gemm_bf16_mi16_body(const GemmArgs& g, uint8_t* 
                 "epilogue class");
   static_assert(!staged_act(ACT) || (BM == 256 && BN == 256 && NW == 8 && !RAGGED),
                 "other epilogues: whole 256 x 256 tiles");
-  static_assert(!RAGGED || LB == L_KCONTIG || LB == L_RCONTIG, "ragged tiles: B [N, K] or [K, N]");
   // Tiles: 256 x 256 with eight waves of 128 x 64; 128 x 128 with four of
   // 64 x 64; 256 x 128 with eight of 128 x 32.
   static_assert((BM == 256 && BN == 256 && NW == 8) || (BM == 128 && BN == 128 && NW == 4) ||
                     (BM == 256 && BN == 128 && NW == 8),
                 "256 x 256 (8 waves), 128 x 128 (4 waves) or 256 x 128 (8 waves)");
-  static_assert(BN == 256 || LB == L_KCONTIG || LB == L_RCONTIG, "packed B: 256-column tiles");
+  // Packed B (its padded columns a whole number of tiles, K of stages): ragged
+  // for M, and N up to the padding.
   static_assert(S == 2 || (S == 4 && BM == 128 && BN == 128 && !staged_act(ACT)), "stages: 2, or 4 of 128 x 128");
   typedef float f32x4_t __attribute__((ext_vector_type(4)));
   // Packed B as in gemm_bf16_dma64_kernel: K-major panels and 32 x 32 blocks
@@ -125,7 +125,7 @@ __device__ __forceinline__ void gemm_bf16_mi16_body(const GemmArgs& g, uint8_t* 
     for (int q = 0; q < LA; ++q) va[q] = kc_voff_clamped(g.a.ld, m0 + wave * (BM / NW) + q * 8 + rr, g.m, q & 1);
     if constexpr (!BT) {
 #pragma unroll
-      for (int q = 0; q < LBN; ++q)
+      for (int q = 0; q < (LB == L_KCONTIG ? LBN : 0); ++q)
         vb[q] = kc_voff_clamped(g.b.ld, n0 + wave * (BN / NW) + q * 8 + rr, g.n, q & 1);
     }
   }
@@ -140,7 +140,8 @@ __device__ __forceinline__ void gemm_bf16_mi16_body(const GemmArgs& g, uint8_t* 
     // bytes: slabs of 4 KiB, one per K pair kp = 16 ks + 4 f + i (i, ks
     // outer), each holding the tile's 16 groups of 16 columns as 256-byte
     // lines [f 4][16 columns][K pair]. 1 KiB load b (of the stage's 32) fills
-    // slab (ks, i) = (b / 16, b / 4 % 4), groups 4 (b % 4) .. + 3; lane l
+    // slab (ks, i) = (b / 16, b / 4 % 4), groups 4 (b % 4) .. + 3 (128-column
+    // tiles: slabs of 2 KiB, two loads each); lane l
     // takes group 4 (b % 4) + l / 16, f = l / 4 % 4, columns 4 (l % 4) .. + 3,
     // i.e. K-pair row 16 ks + 4 f + i of tile columns 64 (b % 4) + lam,
     // lam = 16 (l / 16) + 4 (l % 4). Every load still reads 8 whole 128-byte
@@ -154,22 +155,31 @@ __device__ __forceinline__ void gemm_bf16_mi16_body(const GemmArgs& g, uint8_t* 
     soff_b = blk_b = 0;
 #pragma unroll
     for (int q = 0; q < LBN; ++q) {
-      const int b = wave * LBN + q, ks = b >> 4, i = (b >> 2) & 3;
-      const int64_t col = n0 + 64 * (b & 3);
+      constexpr int CG = BN / 64;  // loads per slab
+      const int b = wave * LBN + q, ks = b / (4 * CG), i = (b / CG) & 3;
+      const int64_t col = n0 + 64 * (b % CG);
       vn_off[q] = (int32_t)((16 * ks + i) * 4 * P + (col / P) * (g.b.kpad / 2) * 4 * P + (col % P) * 4);
     }
   } else if constexpr (BPK) {
     // Element (k, n) at col(n) + row(k); a lane's 8 columns stay in one panel
     // or block, the lane offset holds col(n) and the row within the K pair.
     // Rows 8 w .. 8 w + 7: bit 3 of the row is the wave's parity.
-    const int r = lane >> 5, c = (lane & 31) ^ (((wave * (64 / NW)) >> 2) & 2);
+    // (128-column tiles: four K rows of 256 bytes per load, as row-major B.)
     auto col = [&](int64_t n) -> int64_t {
       if constexpr (LB == L_PANELS) return (n / P) * g.b.kpad * P + n % P;
       else return (n >> 5) * (g.b.kpad >> 5) * 1024 + (n & 31);
     };
     const int64_t rs = LB == L_PANELS ? P : 32;
-    voff_b0 = (int32_t)((col(n0 + (c ^ swz_n(r)) * 8) + r * rs) * 2);
-    voff_b1 = (int32_t)((col(n0 + (c ^ swz_n(r + 2)) * 8) + r * rs) * 2);
+    const int h = ((wave * (64 / NW)) >> 2) & 2;
+    if constexpr (BN == 128) {
+      const int r = lane >> 4, c = (lane & 15) ^ swz_n(r) ^ h;
+      voff_b0 = (int32_t)((col(n0 + c * 8) + r * rs) * 2);
+      voff_b1 = (int32_t)((col(n0 + (c ^ 2) * 8) + r * rs) * 2);
+    } else {
+      const int r = lane >> 5, c = (lane & 31) ^ h;
+      voff_b0 = (int32_t)((col(n0 + (c ^ swz_n(r)) * 8) + r * rs) * 2);
+      voff_b1 = (int32_t)((col(n0 + (c ^ swz_n(r + 2)) * 8) + r * rs) * 2);
+    }
     soff_b = blk_b = 0;
   } else if constexpr (BT && BN == 128) {
     // 256-byte rows: a 1 KiB load is 4 K rows, lane l filling slot l % 16 of
@@ -260,9 +270,10 @@ __device__ __forceinline__ void gemm_bf16_mi16_body(const GemmArgs& g, uint8_t* 
       lds_dma16(srd_b, voff_b0, vn_off[qb] + (int32_t)((k0 / 2) * 4 * P), sb + qb * 1024);
     } else if constexpr (BPK) {
       const int qb = q - LA;
-      const int64_t kr = k0 + wave * (64 / NW) + 2 * qb;  // even
+      const int64_t kr = k0 + wave * (64 / NW) + (BN == 128 ? 4 : 2) * qb;  // even
       const int64_t row = LB == L_PANELS ? kr * P : (kr >> 5) * 1024 + (kr & 31) * 32;
-      lds_dma16(srd_b, (qb & 1) ? voff_b1 : voff_b0, (int32_t)(row * 2), sb + qb * 1024);
+      const bool hi = BN == 128 ? (qb >> 1) & 1 : qb & 1;
+      lds_dma16(srd_b, hi ? voff_b1 : voff_b0, (int32_t)(row * 2), sb + qb * 1024);
     } else if constexpr (RAGGED && !BT) {
       const int qb = q - LA;
       lds_dma16(srd_b, vb[qb], (int32_t)(k0 * 2), sb + qb * 1024);

@@ -1,0 +1,11 @@
+// The 16x16x32 bf16 GEMM kernel's instantiations for B in 32 x 32 blocks.
+#include "hmx_gemm_mi16_launch.hpp"
+
+namespace hmx {
+
+bool launch_mi16_blocked(const GemmArgs& g, Mi16Tile t, dim3 grid, hipStream_t s) {
+  return g.c_dtype == HMX_DTYPE_BF16 ? mi16_packed<L_BLOCKED, true>(g, t, grid, s)
+                                     : mi16_packed<L_BLOCKED, false>(g, t, grid, s);
+}
+
+}  // namespace hmx

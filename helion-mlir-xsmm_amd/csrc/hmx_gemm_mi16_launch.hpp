@@ -72,6 +72,14 @@ bool mi16_plain(const GemmArgs& g, Mi16Tile t, dim3 grid, hipStream_t s) {
                   : mi16_tile<LB, BF16, false, 128, 128, 4, 2>(g, grid, s);
 }
 
+// Packed B: whole 256 x 256 tiles, or (ragged) M of any size.
+template <int LB, bool BF16>
+bool mi16_packed(const GemmArgs& g, Mi16Tile t, dim3 grid, hipStream_t s) {
+  if (t.bm == 256) return t.ragged ? mi16_tile<LB, BF16, true, 256, 256, 8, 2>(g, grid, s) : mi16_whole<LB, BF16>(g, grid, s);
+  return t.stages == 4 ? mi16_tile<LB, BF16, true, 128, 128, 4, 4>(g, grid, s)
+                       : mi16_tile<LB, BF16, true, 128, 128, 4, 2>(g, grid, s);
+}
+
 template <int LB, bool BF16>
 bool mi16_rounds(const GemmArgs& head, const GemmArgs& rest, unsigned head_blocks, unsigned rest_blocks,
                  hipStream_t s) {
