@@ -324,6 +324,15 @@ int make_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int64_t batch, int 
         big_tiles >= cus)
       pick = -2;
   }
+  // bf16: 256 x 256 tiles that leave some CUs idle, where 128 x 128 ones would
+  // take three rounds or more. A 64-deep stage of the big tile takes ~1.33 us,
+  // of the small one ~0.55 per workgroup on a CU: same box, 128 -> 256, 1024 x
+  // 11008 x 4096 on 32 x 32 blocks 96 -> 82 us (172 big tiles), 3000 x 4096 x 4096
+  // 95 -> 81 (192), 3000^3 with B [N, K] 91 -> 68 (144). Other CU counts, where
+  // this was not measured, keep the rule above.
+  if (bf16 && pick == 1 && tile_m <= 0 && tile_n <= 0 && tile_k <= 0 && !trans_a && k >= 512 && splits <= 1 &&
+      cus == kMi355x.cus && ceil_div(m, 128) * ceil_div(n, 128) * batch > 2 * (int64_t)cus)
+    pick = 0;
   // bf16 packed B on 128 x 128 tiles, where the direct-to-LDS kernel reads it
   // (launches it cannot take go to the 256 x 256 register-staged kernel).
   if (packed && bf16 && (k % 64 != 0 || n % 128 != 0 || program)) pick = 0;
