@@ -382,6 +382,39 @@ int make_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int64_t batch, int 
   return HMX_OK;
 }
 
+// The small f32 kernel (32 x 32 tiles, K split inside the workgroup, no
+// workspace) takes the plain products of few tiles. HIP-graph replay, planned
+// tiles -> this kernel:
+// - one 32 x 32 tile a CU: 512^3 11.9 -> 8.5 us, 256 x 256 x 1024 12.8 -> 11.6,
+//   384 x 384 x 2048 20.8 -> 18.9, 64 x 4096 x 4096 59 -> 35;
+// - two a CU where the plan leaves 128 x 128 tiles half empty or does not split
+//   64 x 64 ones: 32 x 16384 x 4096 167 -> 69, 700 x 700 x 512 22.1 -> 14.7,
+//   640 x 640 x 4096 127 -> 66. Split 64 x 64 tiles are better (64 x 8000 x 4000
+//   52 -> 70, 40 x 8000 x 2000 34 -> 41), so are whole ones of a short K
+//   (64 x 8000 x 256 8.9 -> 12.1), and with more tiles this kernel reads more than
+//   it saves (1000 x 1000 x 300 15.7 -> 26);
+// - not a long K over few workgroups, which is better split over the grid
+//   (256 x 256 x 4096 20 -> 32, 300 x 300 x 3001 26 -> 30), unless at most 32 rows
+//   or columns leave half of each larger tile empty (8 x 4096 x 4096 55 -> 29);
+// - below K = 256 both take the time of a launch (64^3 4.0 -> 4.3).
+// A caller's own splits or tile, or the plan of a limited workspace, keep the plan.
+bool small_f32(const Plan& plan, int ab_dtype, int64_t m, int64_t n, int64_t k, int64_t batch, int trans_a,
+               int b_layout, bool packed, int epilogue, int cus) {
+  if (ab_dtype != HMX_DTYPE_F32 || packed || epilogue == HMX_EPI_PROGRAM || k < 256 || batch >= 65536) return false;
+  const int64_t tiles = ceil_div(m, 32) * ceil_div(n, 32) * batch;
+  if (tiles > 2 * (int64_t)cus) return false;
+  if (k > std::max<int64_t>(1024, (std::min(m, n) <= 32 ? 128 : 16) * tiles)) return false;
+  Plan own;
+  if (make_plan(ab_dtype, m, n, k, batch, trans_a, b_layout, 0, -1, 0, 0, 0, cus, epilogue, own) != HMX_OK ||
+      plan.splits != own.splits || plan.tile.bm != own.tile.bm || plan.tile.bn != own.tile.bn ||
+      plan.tile.bk != own.tile.bk)
+    return false;
+  // The waves keep 16 partial sums in all: no fewer than the plan's splits.
+  if (own.splits > 16) return false;
+  if (tiles <= cus) return true;
+  return own.tile.bm == 128 ? std::min(m, n) <= 64 : own.splits == 1 && (k >= 512 || m % 64 != 0 || n % 64 != 0);
+}
+
 // The direct-to-LDS bf16 kernel serves every case it can unless the
 // environment sets HMX_GEMM_DMA=0 (which selects the register-staged kernel,
 // for comparison).
@@ -575,6 +608,31 @@ int gemm_impl(int ab_dtype, int c_dtype, const void* a, int64_t lda, int trans_a
       }
       return HMX_OK;
     }
+  }
+  // (A workspace short of the plan is refused below, as for the planned launch.)
+  if ((use_scratch || plan.workspace_bytes <= 0 || (workspace && workspace_bytes >= plan.workspace_bytes)) &&
+      small_f32(plan, ab_dtype, m, n, k, batch, trans_a, b_layout, packed, epilogue, dev.cus)) {
+    GemmArgs g{};
+    g.a = Operand{a, lda, m, 0, 0, false, true, 0};
+    g.b = Operand{b, ldb, n, 0, 0, false, true, 0};
+    g.stride_a = stride_a;
+    g.stride_b = stride_b;
+    g.m = m;
+    g.n = n;
+    g.k = k;
+    g.xcds = dev.xcds;
+    g.bias = bias;
+    g.scale = scale;
+    g.shift = shift;
+    g.vec_dtype = vec_dtype;
+    g.act = epilogue;
+    g.act_arg = epilogue_arg;
+    g.c = c;
+    g.c_dtype = c_dtype;
+    g.ldc = ldc;
+    g.stride_c = stride_c;
+    launch_gemm_f32_small(g, trans_a ? L_RCONTIG : L_KCONTIG, lb, batch, (hipStream_t)stream);
+    return check_launch("gemm");
   }
   // Workspace is checked once the launch is known (below): a B transposed or
   // padded up front (plan.bt_bytes), then an A (plan.at_bytes), then

@@ -487,6 +487,10 @@ bool gemm_bf16_dma_packed_ok(const GemmArgs& g, int lb);
 void launch_gemm_f32_dma(const GemmArgs& g, int lb, dim3 grid, hipStream_t s);
 void launch_gemm_f32(const GemmArgs& g, int tile_bm, int la, int lb, bool guard, dim3 grid,
                      hipStream_t s);
+// hmx_gemm_f32_small.hip: f32 on 32 x 32 tiles, K split inside the workgroup; A and
+// B K-contiguous or row-contiguous, any shape and alignment, any epilogue but
+// programs, C bf16 or f32.
+void launch_gemm_f32_small(const GemmArgs& g, int la, int lb, int64_t batch, hipStream_t s);
 void launch_splitk_reduce(const float* partials, int splits, int64_t batch, const GemmArgs& r,
                           bool vec4, hipStream_t s);
 // hmx_jit.cpp: the 16x16x32 kernel (layout lb, bf16 or f32 C, ragged or
