@@ -149,17 +149,19 @@ int auto_splits(TileChoice tile, int64_t tiles, int64_t m, int64_t n, int64_t k,
     const int64_t need = (int64_t)s2 * batch * m * n * 4;
     // The f32 partials' traffic (written once, read once) at most an eighth
     // of the operands'. With `fill`, bf16 128 x 128 tiles of products of at
-    // least 2^30 multiply-adds (rows the direct-to-LDS kernels read) also split while the grid
-    // stays within one workgroup per CU, each chunk keeps 16 or more stages
-    // and the partials move at most the operands' bytes: a grid of one such
-    // workgroup per CU on a few CUs is latency-bound, and filling the CUs
-    // pays for the partials (same box, unsplit -> split: 1024 x 1024 x 4096
-    // 31.5 -> 21.5 us, 512 x 2048 x 8192 57 -> 28.5 us, 256 x 4000 x 4096
-    // 33.7 -> 27.9 us, 768 x 768 x 3072 24.5 -> 20.5 us; a grid past one
-    // workgroup per CU loses the four-stage ring: 256 x 11008 x 4096
-    // 36 -> 44.5 us in two).
+    // least 2^29 multiply-adds (rows the direct-to-LDS kernels read) also split
+    // while the grid stays within one workgroup per CU, each chunk keeps 16 or
+    // more stages and the partials move at most the operands' bytes: a grid of
+    // one such workgroup per CU on a few CUs is latency-bound, and filling the
+    // CUs pays for the partials (same box, unsplit -> split: 1024 x 1024 x 4096
+    // 31.5 -> 21.5 us, 512 x 2048 x 8192 57 -> 28.5, 768 x 768 x 3072 24.5 ->
+    // 20.5, 512 x 512 x 2048 23.9 -> 15.8, 200 x 1000 x 4000 31.8 -> 29.3; a grid past
+    // one workgroup per CU loses the four-stage ring: 256 x 11008 x 4096
+    // 36 -> 44.5 us in two). Smaller products and chunks of 8 stages
+    // gain as well (256 x 256 x 2048 23.8 -> 11.3), but those plans are
+    // fixed: unsplit with no workspace, and 16 stages.
     const bool fills = fill && esz == 2 && tile.bm == 128 && kt / s2 >= 16 && tiles * s2 <= cus &&
-                       (double)batch * m * n * k >= 1073741824.0 && need <= operand_bytes;
+                       (double)batch * m * n * k >= 536870912.0 && need <= operand_bytes;
     if ((max_ws >= 0 && need > max_ws) || (2 * need > operand_bytes / 4 && !fills)) break;
     splits = s2;
   }
