@@ -231,9 +231,15 @@ const char* hmx_jit_last_log(void);
  * kernel's own 32 x 32 x 64) take a skinny kernel: one workgroup per 32
  * columns of C, K split over its waves and summed in a fixed order, no
  * workspace (hmx_gemm_plan reports tile 32 x 32 x 64). The workspace also
- * takes a bf16 operand the library transposes once before the product (a
- * row-major B with ragged K, an A stored [K, M] of 512 or more rows, columns
- * and K); hmx_gemm_plan counts it. A row-major A or a B [N, K] spanning 2^31
+ * takes a bf16 operand the library prepares once before the product: rows of
+ * an odd number of elements are copied with padding, an A stored [K, M] of 512
+ * or more rows, columns and K is transposed, and so is a row-major B that no
+ * kernel reads in place (its bytes are planned by shape, and unused where the
+ * launch can read it). hmx_gemm_plan counts it. At most 32 rows of A against
+ * a packed bf16 B take a streaming kernel (tile 32 x 64 x 32), and small f32
+ * products planned as split or partial tiles run as one kernel of 32 x 32
+ * tiles that leaves the workspace alone, unless the caller names other splits
+ * or another tile. A row-major A or a B [N, K] spanning 2^31
  * bytes or more runs as one launch per block of whole tiles.
  * Stands in for matmul (helion_mlir_utils/matmul.py:1446-1570), its
  * fused-pack kernel (259-328), the f32 fused and blocked kernels (156-228,
