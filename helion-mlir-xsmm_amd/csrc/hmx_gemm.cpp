@@ -271,9 +271,19 @@ int make_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int64_t batch, int 
   plan.pad_b = pads && (b_layout == HMX_B_TRANS ? k % 2 != 0 : n % 2 != 0) && b_elems * 2 < INT32_MAX;
   plan.at_bytes = plan.transpose_a || plan.pad_a ? ceil_div(batch * m * k8 * 2, 256) * 256 : 0;
   plan.bt_bytes = plan.pad_b ? ceil_div(batch * b_elems * 2, 256) * 256 : 0;
-  if (max_ws >= 0 && plan.at_bytes + plan.bt_bytes > max_ws) {
-    plan.transpose_a = plan.pad_a = plan.pad_b = false;
-    plan.at_bytes = plan.bt_bytes = 0;
+  // Padded copies only take what the partials of the caller's own splits, or of
+  // a program no kernel runs fused (K not in whole stages), leave of the
+  // workspace: a workspace of just those keeps its launch, without the copies.
+  const int64_t own_partials =
+      splits > 1 || (program && k % 64 != 0) ? (int64_t)std::max(splits, 1) * batch * m * n * 4 : 0;
+  if (max_ws >= 0 && (plan.pad_a || plan.pad_b) && plan.at_bytes + plan.bt_bytes + own_partials > max_ws) {
+    plan.pad_a = plan.pad_b = false;
+    if (!plan.transpose_a) plan.at_bytes = 0;
+    plan.bt_bytes = 0;
+  }
+  if (max_ws >= 0 && plan.at_bytes > max_ws) {
+    plan.transpose_a = false;
+    plan.at_bytes = 0;
   }
   if (plan.transpose_a) trans_a = 0;
   if (max_ws >= 0) max_ws -= plan.at_bytes + plan.bt_bytes;

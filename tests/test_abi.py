@@ -308,6 +308,22 @@ def test_program_epilogues_plan_their_partials(lib: ctypes.CDLL) -> None:
     assert _plan(lib, bf16, 4096, 4096, 4096, epi=native.EPI_GELU) == (1, 256, 256, 64, 0)
 
 
+@pytest.mark.parametrize("layout", [native.B_ROW, native.B_TRANS])
+@pytest.mark.parametrize(("m", "n", "k"), [(100, 101, 501), (64, 64, 4097), (600, 333, 129)])
+def test_padded_copies_take_what_the_partials_leave(lib: ctypes.CDLL, layout: int, m: int, n: int, k: int) -> None:
+    # Odd rows are copied with padding where the workspace holds the copies and
+    # the partials; one that holds the caller's own splits' partials and no more
+    # (what the header asks for), or a staged program's, plans no copy.
+    bf16 = native.DTYPE_BF16
+    for splits, epi in [(2, native.EPI_IDENTITY), (4, native.EPI_IDENTITY), (1, native.EPI_PROGRAM)]:
+        s, *_, ws = _plan(lib, bf16, m, n, k, splits=splits, b_layout=layout, epi=epi)
+        partials = s * m * n * 4
+        assert ws > partials
+        for room in (partials, (partials + ws) // 2, ws - 1):
+            assert _plan(lib, bf16, m, n, k, splits=s, max_ws=room, b_layout=layout, epi=epi)[4] <= room
+        assert _plan(lib, bf16, m, n, k, splits=s, max_ws=ws, b_layout=layout, epi=epi)[4] == ws
+
+
 @pytest.mark.parametrize("epi", [native.EPI_IDENTITY, native.EPI_PROGRAM])
 @pytest.mark.parametrize("cus", [256, 304, 80, 32])
 @pytest.mark.parametrize("ab", [native.DTYPE_BF16, native.DTYPE_F32])
